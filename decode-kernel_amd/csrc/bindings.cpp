@@ -107,11 +107,15 @@ torch::Tensor gemv_common(torch::Tensor packed, torch::Tensor scales, torch::Ten
     ws_ptr = workspace.data_ptr();
   }
 
-  const int rc = dk_w4a16_gemv(reinterpret_cast<const uint32_t*>(packed.data_ptr<int32_t>()),
-                               reinterpret_cast<const uint16_t*>(scales.data_ptr<at::Half>()),
-                               reinterpret_cast<const uint16_t*>(x.data_ptr<at::Half>()),
-                               reinterpret_cast<uint16_t*>(y.data_ptr<at::Half>()), M, K, B, &cfg,
-                               ws_ptr, ws_bytes, current_stream(x));
+  // Batches take dk_w4a16_linear, which has the many-batch kernel too.
+  const auto* pp = reinterpret_cast<const uint32_t*>(packed.data_ptr<int32_t>());
+  const auto* sp = reinterpret_cast<const uint16_t*>(scales.data_ptr<at::Half>());
+  const auto* xp = reinterpret_cast<const uint16_t*>(x.data_ptr<at::Half>());
+  auto* yp = reinterpret_cast<uint16_t*>(y.data_ptr<at::Half>());
+  const int rc = reuse_weights ? dk_w4a16_linear(pp, sp, xp, yp, M, K, B, ws_ptr, ws_bytes,
+                                                 current_stream(x))
+                               : dk_w4a16_gemv(pp, sp, xp, yp, M, K, B, &cfg, ws_ptr, ws_bytes,
+                                               current_stream(x));
   check_status(rc, "w4a16_gemv");
   return y;
 }

@@ -23,6 +23,7 @@
 #include <string>
 #include <type_traits>
 
+#include "dk_gemm.hpp"
 #include "dk_host.hpp"
 #include "dk_kernels.hpp"
 #include "dk_mlp.hpp"
@@ -438,6 +439,115 @@ int launch_v5(const Launch& L, const uint4* p, const uint16_t* s, const uint4* x
 }
 #undef DK_BATCH
 
+// The many-batch kernel (gemm_w4): WMN x WKN waves, 32 NBT batch rows per
+// workgroup; wmn = 0: not this kernel.
+struct GemmShape {
+  int wmn = 0, wkn = 0, nbt = 0;
+};
+
+long long ceil_div(long long a, long long b) { return (a + b - 1) / b; }
+
+// The shape with the least estimated time for M rows, `unit` of them per wave
+// (64; 32 of each matrix for gate/up). A workgroup takes fixed + step us per
+// step (one group per K part); eight-wave workgroups run one to a CU, in
+// rounds of 256; four-wave ones two to a CU when there are more than 256, a
+// pair then taking `pair` us per step. Fitted to the seven shapes' times over
+// 15 (M, K) from 512 x 4096 to 28672 x 8192 and six of gate/up, at 15 batches
+// from 17 to 1000: the choice is 0.1% from the best shape on average and 5% at
+// worst. What decides is the number of workgroups: few take many K parts and
+// few batch rows each, many decode each weight for 128 batch rows and leave
+// the CU to two workgroups (us, the choice first; 4096 x 4096, B = 64 10.8 for
+// <1, 8, 1>, 13.9 for <1, 8, 2>, 19.7 for <2, 4, 2>; B = 1000 38.2 for
+// <2, 4, 4>, 42.3 for <1, 4, 4>, 49.6 for <1, 8, 4>, 64.4 for <4, 1, 4>; 28672
+// x 8192, B = 2048 820 for <4, 1, 4>, 972 for <2, 4, 4>).
+GemmShape gemm_best(int M, int K, int B, int unit) {
+  struct Cand {
+    int wmn, wkn, nbt;
+    double fixed, step, pair;
+  };
+  constexpr Cand kCands[] = {
+      {1, 8, 1, 3.8, 2.0, 0.0}, {1, 8, 2, 4.0, 3.0, 0.0}, {2, 4, 2, 4.3, 2.36, 0.0},
+      {1, 8, 4, 5.4, 4.6, 0.0}, {2, 4, 4, 6.2, 3.74, 0.0}, {1, 4, 4, 3.7, 2.95, 4.1},
+      {4, 1, 4, 3.0, 2.1, 3.47},
+  };
+  const int G = K / DK_GROUP_SIZE;
+  GemmShape best;
+  double best_us = 0.0;
+  for (const Cand& c : kCands) {
+    const long long n = ceil_div(M, unit * c.wmn) * ceil_div(B, 32 * c.nbt);
+    if (n > 0x7fffffffLL) continue;
+    const double steps = (double)ceil_div(G, c.wkn);
+    double us;
+    if (c.wmn * c.wkn == 8) {
+      us = (double)ceil_div(n, 256) * (c.fixed + steps * c.step);
+    } else {
+      const long long rest = n % 512;
+      us = (double)(n / 512) * (c.fixed + steps * c.pair) +
+           (rest ? c.fixed + steps * (rest > 256 ? c.pair : c.step) : 0.0);
+    }
+    if (best.wmn == 0 || us < best_us) {
+      best = {c.wmn, c.wkn, c.nbt};
+      best_us = us;
+    }
+  }
+  return best;
+}
+
+// Where gemm_w4 takes the weight-reuse path's batches (`pairs`: the scales
+// load in pairs) and gate/up's: above 16 batch rows, where its workgroups,
+// 64 rows by 32-128 batch rows each, fill half the chip. Its 32-bit offsets
+// take K up to 2^21. Against the 16-row tiles (us, gemm_w4 first):
+//   pairs:  M = K = 4096, B = 64 10.8 (9.3), 96 13.8 (14.1), 192 14.4 (21.7);
+//           M = 2048, K = 11008, B = 128 29.8 (18.7), 256 30.8 (31.1), 512 47.7 (51.4);
+//           M = 1024, K = 8192, B = 512 24 (25.7), 1000 37.9 (41.2);
+//           M = 8192, K = 28672, B = 32 53.4 (46.5), 48 51.5 (69.2);
+//           M = 11008, K = 4096, B = 17 11.0 (14.4);
+//           rows of up to 1024 weights stay (M = 4096, K = 1024, B = 64 5.3
+//           (4.7), 128 6.7 (6.7), 256 6.9 (8.7))
+//   no pairs (the 16-row tiles then cost the same for every 16 batch rows):
+//           M = 4096, K = 4224, B = 32 10.7 (7.7), 64 11.1 (13.4);
+//           M = 512, K = 4224, B = 256 13.1 (10.4), 512 14.6 (20.0)
+//   gate/up, likewise:
+//           I = 2048, H = 4096, B = 64 11.0 (10.2), 128 15.7 (17.7);
+//           I = 3584, H = 8192, B = 32 18.3 (19.9), 48 18.5 (28.1);
+//           I = 11008, H = 4096, B = 16 20.5 (16.0), 17 20.3 (23.6)
+GemmShape gemm_shape(int M, int K, int B, bool pairs) {
+  if (B <= 16 || K > (1 << 21)) return {};
+  const bool take =
+      pairs ? K > 1024 && (M > 8192 || (B > 32 && ceil_div(M, 64) * ceil_div(B, 64) >= 128))
+            : ceil_div(M, 16) * ceil_div(B, 16) > 512;
+  return take ? gemm_best(M, K, B, 64) : GemmShape{};
+}
+
+GemmShape gate_up_gemm_shape(int I, int H, int B) {
+  if (B <= 16 || H > (1 << 21) || ceil_div(I, 16) * ceil_div(B, 16) <= 512) return {};
+  return gemm_best(I, H, B, 32);
+}
+
+template <int WMN, int WKN, int NBT, bool kGateUp>
+int launch_gemm_t(const Launch& L, const char* what, const uint4* w0, const uint16_t* s0,
+                  const uint4* w1, const uint16_t* s1, const uint4* x, uint16_t* y, int M, int K,
+                  int B) {
+  const long long n = ceil_div(M, (kGateUp ? 32 : 64) * WMN) * ceil_div(B, 32 * NBT);
+  return L(what, dk::gemm_w4<WMN, WKN, NBT, kGateUp>, dim3((unsigned)n), dim3(WMN * WKN * 64), 0,
+           w0, s0, w1, s1, x, y, M, K, B);
+}
+
+template <bool kGateUp>
+int launch_gemm(const Launch& L, const GemmShape& g, const uint4* w0, const uint16_t* s0,
+                const uint4* w1, const uint16_t* s1, const uint4* x, uint16_t* y, int M, int K,
+                int B) {
+  const char* what = kGateUp ? "gate/up launch" : "reuse launch";
+#define DK_GEMM(m, k, n)                            \
+  if (g.wmn == m && g.wkn == k && g.nbt == n)       \
+    return launch_gemm_t<m, k, n, kGateUp>(L, what, w0, s0, w1, s1, x, y, M, K, B);
+  DK_GEMM(1, 8, 1) DK_GEMM(1, 8, 2) DK_GEMM(2, 4, 2) DK_GEMM(1, 8, 4) DK_GEMM(2, 4, 4)
+  DK_GEMM(1, 4, 4) DK_GEMM(4, 1, 4)
+#undef DK_GEMM
+  return fail(DK_ERR_UNSUPPORTED, "internal: no kernel for %d x %d waves, %d batch tiles", g.wmn,
+              g.wkn, g.nbt);
+}
+
 // Batches that the MFMA tiles take on the fused gate/up step. Tiles against
 // the streaming kernel's batch tiles in brackets (us per launch, both
 // matrices; 8 waves, blocks of two groups, chosen over 4 or 16 waves with
@@ -517,9 +627,12 @@ int launch_gate_up_lds_t(const Launch& L, const uint4* g, const uint16_t* gs, co
 int launch_gate_up(const Launch& L, const uint4* g, const uint16_t* gs, const uint4* u,
                    const uint16_t* us, const uint4* x, uint16_t* h, int I, int H, int B) {
   const bool pairs = (H / DK_GROUP_SIZE) % 2 == 0 && aligned(gs, 4) && aligned(us, 4);
+  const GemmShape gemm = gate_up_gemm_shape(I, H, B);
+  if (gemm.wmn) return launch_gemm<true>(L, gemm, g, gs, u, us, x, h, I, H, B);
   if (gate_up_tiles(I, H, B, pairs)) {
     const dim3 grid((I + 15) / 16, (B + dk::kReuseBatch - 1) / dk::kReuseBatch);
-    // From 8 batch rows, both tiles' operands staged in LDS (as the GEMV's
+    // (Above 16 batch rows only where gate_up_gemm_shape leaves them.) From 8
+    // batch rows, both tiles' operands staged in LDS (as the GEMV's
     // gemv_reuse_lds), 8 waves up to I = 4096 and 16 batch rows, else 4
     // (us, against the tiles that load the operands directly):
     //                        B = 8           B = 16          B = 32
@@ -1004,9 +1117,10 @@ int check_io(const uint32_t* packed, const uint16_t* scales, const uint16_t* x, 
   return DK_OK;
 }
 
+// many: the reuse path's batches may run on gemm_w4 (dk_w4a16_linear).
 int gemv_impl(const uint32_t* packed, const uint16_t* scales, const uint16_t* x, uint16_t* y, int M,
               int K, int B, const dk_gemv_config* cfg, void* workspace, size_t workspace_bytes,
-              const Launch& L) {
+              const Launch& L, bool many = false) {
   int rc = dk_gemv_validate(M, K, B, cfg);
   if (rc != DK_OK) return rc;
   if (M <= 0 || K <= 0 || B <= 0) return DK_OK;
@@ -1030,6 +1144,10 @@ int gemv_impl(const uint32_t* packed, const uint16_t* scales, const uint16_t* x,
 
   if (cfg->reuse_weights) {
     const bool pairs = (K / DK_GROUP_SIZE) % 2 == 0 && aligned(scales, 4);
+    const GemmShape gemm = many ? gemm_shape(M, K, B, pairs) : GemmShape{};
+    if (gemm.wmn)
+      return L.stamp(launch_gemm<false>(L, gemm, p4, scales, nullptr, nullptr, x4, y, M, K, B),
+                     DK_STAMP_REUSE);
     if (reuse_shape(M, K, B, pairs) == ReuseShape::kStream)
       return L.stamp(launch_v5<dk::LayoutLogical, DK_STAMP_REUSE>(L, p4, scales, x4, y, M, K, B),
                      DK_STAMP_REUSE);
@@ -1186,6 +1304,16 @@ int dk_w4a16_gemv(const uint32_t* packed, const uint16_t* scales, const uint16_t
   return gemv_impl(packed, scales, x, y, M, K, B, cfg, workspace, workspace_bytes, Launch{stream});
 }
 
+int dk_w4a16_linear(const uint32_t* packed, const uint16_t* scales, const uint16_t* x, uint16_t* y,
+                    int M, int K, int B, void* workspace, size_t workspace_bytes,
+                    hipStream_t stream) {
+  dk_gemv_config cfg;
+  dk_gemv_config_default(&cfg);
+  cfg.reuse_weights = 1;
+  return gemv_impl(packed, scales, x, y, M, K, B, &cfg, workspace, workspace_bytes, Launch{stream},
+                   true);
+}
+
 int dk_w4a16_gemv_noalloc(const uint32_t* packed, const uint16_t* scales, const uint16_t* x,
                           uint16_t* y, int M, int K, int B, const dk_gemv_config* cfg,
                           hipStream_t stream) {
@@ -1213,8 +1341,8 @@ int dk_w4a16_gemv_ref_workspace(const uint32_t* packed, const uint16_t* scales, 
   return gemv_ref_workspace_impl(packed, scales, x, y, M, K, B, cfg, workspace, Launch{stream});
 }
 
-int dk_gemv_describe(int M, int K, int B, const dk_gemv_config* cfg, size_t workspace_bytes,
-                     dk_launch_info* info) {
+static int describe(int M, int K, int B, const dk_gemv_config* cfg, size_t workspace_bytes,
+                    bool many, dk_launch_info* info) {
   if (!info) return fail(DK_ERR_INVALID_ARGUMENT, "info must not be NULL");
   *info = dk_launch_info{};
   // Placeholder addresses with every alignment the checks ask for; in
@@ -1223,7 +1351,30 @@ int dk_gemv_describe(int M, int K, int B, const dk_gemv_config* cfg, size_t work
   const auto* h = reinterpret_cast<const uint16_t*>(uintptr_t{4096});
   void* ws = workspace_bytes > 0 ? reinterpret_cast<void*>(uintptr_t{4096}) : nullptr;
   Launch L{nullptr, info};
-  return gemv_impl(p, h, h, const_cast<uint16_t*>(h), M, K, B, cfg, ws, workspace_bytes, L);
+  return gemv_impl(p, h, h, const_cast<uint16_t*>(h), M, K, B, cfg, ws, workspace_bytes, L, many);
+}
+
+int dk_gemv_describe(int M, int K, int B, const dk_gemv_config* cfg, size_t workspace_bytes,
+                     dk_launch_info* info) {
+  return describe(M, K, B, cfg, workspace_bytes, false, info);
+}
+
+int dk_linear_describe(int M, int K, int B, size_t workspace_bytes, dk_launch_info* info) {
+  dk_gemv_config cfg;
+  dk_gemv_config_default(&cfg);
+  cfg.reuse_weights = 1;
+  return describe(M, K, B, &cfg, workspace_bytes, true, info);
+}
+
+int dk_gate_up_describe(int I, int H, int B, dk_launch_info* info) {
+  if (!info) return fail(DK_ERR_INVALID_ARGUMENT, "info must not be NULL");
+  *info = dk_launch_info{};
+  const auto* p = reinterpret_cast<const uint4*>(uintptr_t{4096});
+  const auto* h = reinterpret_cast<const uint16_t*>(uintptr_t{4096});
+  if (I <= 0 || H <= 0 || B <= 0) return DK_OK;
+  if (H % DK_GROUP_SIZE != 0)
+    return fail(DK_ERR_INVALID_ARGUMENT, "H=%d must be divisible by group size 128", H);
+  return launch_gate_up(Launch{nullptr, info}, p, h, p, h, p, const_cast<uint16_t*>(h), I, H, B);
 }
 
 int dk_last_kernel_stamp(void) {
@@ -1327,7 +1478,7 @@ int dk_mlp_decode(const uint32_t* gate_packed, const uint16_t* gate_scales,
   const bool with_split = down_ws > 0 && workspace_bytes >= mlp_h_bytes(I, B) + down_ws;
   void* ws = with_split ? static_cast<char*>(workspace) + mlp_h_bytes(I, B) : nullptr;
   return gemv_impl(down_packed, down_scales, h, y, H, I, B, &cfg, ws, with_split ? down_ws : 0,
-                   Launch{stream});
+                   Launch{stream}, B > 1);
 }
 
 const char* dk_last_error(void) { return dk::g_err.c_str(); }

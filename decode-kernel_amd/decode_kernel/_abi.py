@@ -74,6 +74,18 @@ _SIGNATURES = {
         [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.POINTER(GemvConfig), ctypes.c_size_t,
          ctypes.POINTER(LaunchInfo)],
     ),
+    "dk_w4a16_linear": (
+        ctypes.c_int,
+        [_P, _P, _P, _P, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P, ctypes.c_size_t, _P],
+    ),
+    "dk_linear_describe": (
+        ctypes.c_int,
+        [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_size_t, ctypes.POINTER(LaunchInfo)],
+    ),
+    "dk_gate_up_describe": (
+        ctypes.c_int,
+        [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.POINTER(LaunchInfo)],
+    ),
     "dk_quantize_pack_f32": (ctypes.c_int, [_P, ctypes.c_int, ctypes.c_int, _P, _P, _P]),
     "dk_repack_paired": (ctypes.c_int, [_P, _P, ctypes.c_int, ctypes.c_int, _P]),
     "dk_unpack_paired": (ctypes.c_int, [_P, _P, ctypes.c_int, ctypes.c_int, _P]),
@@ -140,8 +152,28 @@ def describe(lib: ctypes.CDLL, m: int, k: int, b: int, workspace_bytes: int | No
     info = LaunchInfo()
     check(lib, lib.dk_gemv_describe(m, k, b, ctypes.byref(cfg), workspace_bytes,
                                     ctypes.byref(info)))
+    return _launch(info)
+
+
+def _launch(info: LaunchInfo) -> dict:
     return {"kernel": info.kernel.decode(), "grid": list(info.grid), "block": list(info.block),
             "launches": info.launches}
+
+
+def describe_linear(lib: ctypes.CDLL, m: int, k: int, b: int) -> dict:
+    """The same for dk_w4a16_linear, with the workspace the torch binding passes."""
+    cfg = default_config(lib, reuse_weights=1)
+    ws = lib.dk_gemv_workspace_bytes(m, k, b, ctypes.byref(cfg))
+    info = LaunchInfo()
+    check(lib, lib.dk_linear_describe(m, k, b, ws, ctypes.byref(info)))
+    return _launch(info)
+
+
+def describe_gate_up(lib: ctypes.CDLL, i: int, h: int, b: int) -> dict:
+    """The kernel dk_gate_up_silu would launch."""
+    info = LaunchInfo()
+    check(lib, lib.dk_gate_up_describe(i, h, b, ctypes.byref(info)))
+    return _launch(info)
 
 
 def check(lib: ctypes.CDLL, status: int) -> None:

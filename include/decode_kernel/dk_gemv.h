@@ -121,6 +121,16 @@ int dk_w4a16_gemv(const uint32_t* packed, const uint16_t* scales,
                   const dk_gemv_config* cfg, void* workspace,
                   size_t workspace_bytes, hipStream_t stream);
 
+/* The quantized F.linear for any number of batch rows: what w4a16_linear
+ * (python/decode_kernel/__init__.py:62-83) computes for a batch. Arguments,
+ * checks, optional workspace, stamp and results as dk_w4a16_gemv with
+ * reuse_weights; above 16 batch rows it also has the many-batch kernel, which
+ * decodes each weight once for up to 128 batch rows, and takes it where its
+ * grid fills the chip. */
+int dk_w4a16_linear(const uint32_t* packed, const uint16_t* scales, const uint16_t* x,
+                    uint16_t* y, int M, int K, int B, void* workspace, size_t workspace_bytes,
+                    hipStream_t stream);
+
 /* Size of the per-GPU device array behind dk_w4a16_gemv_noalloc. */
 #define DK_NOALLOC_SCRATCH_BYTES ((size_t)512 << 10)
 
@@ -166,6 +176,9 @@ typedef struct dk_launch_info {
 
 int dk_gemv_describe(int M, int K, int B, const dk_gemv_config* cfg, size_t workspace_bytes,
                      dk_launch_info* info);
+
+/* The same for dk_w4a16_linear. */
+int dk_linear_describe(int M, int K, int B, size_t workspace_bytes, dk_launch_info* info);
 
 /* Kernel-native "paired" weight layout: the same two's-complement int4
  * nibbles and scales, with each word's nibbles permuted so that q_{2j} is at

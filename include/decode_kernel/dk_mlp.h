@@ -22,6 +22,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "decode_kernel/dk_gemv.h" /* dk_launch_info */
+
 #ifdef __cplusplus
 extern "C" {
 #endif
@@ -35,6 +37,10 @@ int dk_gate_up_silu(const uint32_t* gate_packed, const uint16_t* gate_scales,
                     const uint32_t* up_packed, const uint16_t* up_scales,
                     const uint16_t* x, uint16_t* h, int I, int H, int B,
                     hipStream_t stream);
+
+/* The kernel dk_gate_up_silu would launch for aligned operands, without
+ * launching it (see dk_gemv_describe). */
+int dk_gate_up_describe(int I, int H, int B, dk_launch_info* info);
 
 /* Bytes of workspace dk_mlp_decode takes (0 if empty): h, B * I fp16 padded
  * to 256 bytes, then the down projection's split-K workspace where its
