@@ -180,6 +180,31 @@ std::vector<torch::Tensor> quantize_and_pack(torch::Tensor w) {
   return {packed, scales};
 }
 
+// W = q * scale [M, K] in fp32 or fp16. Reference:
+// python/decode_kernel/quantize.py:66-78.
+torch::Tensor dequantize(torch::Tensor packed, torch::Tensor scales, bool fp16) {
+  TORCH_CHECK(packed.is_cuda() && scales.is_cuda() && packed.device() == scales.device(),
+              "packed and scales must be CUDA tensors on one device");
+  TORCH_CHECK(packed.scalar_type() == torch::kInt32, "packed must be int32 (uint32 bit pattern)");
+  TORCH_CHECK(scales.scalar_type() == torch::kFloat16, "scales must be fp16");
+  TORCH_CHECK(packed.dim() == 2 && scales.dim() == 2 && packed.is_contiguous() &&
+                  scales.is_contiguous(),
+              "packed [M,K/8] and scales [M,K/128] must be contiguous");
+  const int64_t M = packed.size(0), K = packed.size(1) * kNibblesPerWord;
+  TORCH_CHECK(K % kGroupSize == 0, "K must be divisible by group size 128");
+  TORCH_CHECK(scales.size(0) == M && scales.size(1) == K / kGroupSize,
+              "scales shape must be [M, K/128]");
+  TORCH_CHECK(M <= INT32_MAX && K <= INT32_MAX, "M and K must fit in int32");
+  c10::DeviceGuard guard(packed.device());
+  auto out = torch::empty({M, K}, scales.options().dtype(fp16 ? torch::kFloat16 : torch::kFloat32));
+  check_status(dk_dequantize(reinterpret_cast<const uint32_t*>(packed.data_ptr<int32_t>()),
+                             reinterpret_cast<const uint16_t*>(scales.data_ptr<at::Half>()),
+                             static_cast<int>(M), static_cast<int>(K), fp16 ? 1 : 0,
+                             out.data_ptr(), current_stream(packed)),
+               "dequantize");
+  return out;
+}
+
 int stream_recommended_blocks() {
   const int blocks = dk_stream_recommended_blocks();
   TORCH_CHECK(blocks > 0, "stream_recommended_blocks failed: ", dk_last_error());
@@ -335,6 +360,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("quantize_and_pack", &quantize_and_pack,
         "fp32 W [M, K] -> (packed int32 [M, K/8], scales fp16 [M, K/128]) on the GPU",
         py::arg("w"));
+  m.def("dequantize", &dequantize, "W = q * scale [M, K] in fp32 or fp16", py::arg("packed"),
+        py::arg("scales"), py::arg("fp16") = false);
   m.def("gate_up_silu", &gate_up_silu,
         "Fused MLP gate/up projection: fp16(silu(gate x) * (up x)) -> [B, I]", py::arg("gate"),
         py::arg("gate_scales"), py::arg("up"), py::arg("up_scales"), py::arg("x"));

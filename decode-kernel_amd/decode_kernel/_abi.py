@@ -87,6 +87,7 @@ _SIGNATURES = {
         [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.POINTER(LaunchInfo)],
     ),
     "dk_quantize_pack_f32": (ctypes.c_int, [_P, ctypes.c_int, ctypes.c_int, _P, _P, _P]),
+    "dk_dequantize": (ctypes.c_int, [_P, _P, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P, _P]),
     "dk_repack_paired": (ctypes.c_int, [_P, _P, ctypes.c_int, ctypes.c_int, _P]),
     "dk_unpack_paired": (ctypes.c_int, [_P, _P, ctypes.c_int, ctypes.c_int, _P]),
     "dk_w4a16_gemv_paired": (

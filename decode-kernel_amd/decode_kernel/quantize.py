@@ -22,6 +22,7 @@ use the torch formulation below on either device.
 from __future__ import annotations
 
 import torch
+import torch.autograd.forward_ad as fwAD
 
 GROUP_SIZE = 128
 NIBBLES_PER_WORD = 8
@@ -106,6 +107,33 @@ def unpack_to_int(packed: torch.Tensor) -> torch.Tensor:
     return q.reshape(m, words * NIBBLES_PER_WORD).to(torch.int32)
 
 
+def _plain_gpu(packed: torch.Tensor, scales: torch.Tensor):
+    """The extension if it can take these tensors with nothing lost, else None."""
+    if not {type(packed), type(scales)} <= {torch.Tensor, torch.nn.Parameter}:
+        return None  # other subclasses (fake tensors) keep their own dispatch
+    if torch.compiler.is_compiling() or torch.jit.is_tracing():
+        return None
+    if torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack():
+        return None
+    wrapped = torch._C._functorch.is_functorch_wrapped_tensor
+    if wrapped(packed) or wrapped(scales) or scales.is_neg():
+        return None
+    if (scales.requires_grad and torch.is_grad_enabled()) or fwAD.unpack_dual(scales).tangent is not None:
+        return None
+    if not (packed.is_cuda and packed.dtype == torch.int32 and packed.dim() == 2
+            and packed.is_contiguous() and packed.shape[1] % (GROUP_SIZE // NIBBLES_PER_WORD) == 0):
+        return None
+    m, groups = packed.shape[0], packed.shape[1] * NIBBLES_PER_WORD // GROUP_SIZE
+    if not (scales.device == packed.device and scales.dtype == torch.float16
+            and scales.shape == (m, groups) and scales.is_contiguous() and m * groups > 0):
+        return None
+    try:
+        from . import _cuda
+    except ImportError:  # as before the extension is built
+        return None
+    return _cuda
+
+
 def dequantize(
     packed: torch.Tensor,
     scales: torch.Tensor,
@@ -114,8 +142,25 @@ def dequantize(
 ) -> torch.Tensor:
     """Materialise W = q * scale [M, K] (for checks; the kernels never do this).
 
-    Reference: python/decode_kernel/quantize.py:66-78.
+    Reference: python/decode_kernel/quantize.py:66-78. GPU tensors in the
+    kernels' own format go through one HIP pass, with the bits of the torch
+    formulation below; everything else, and everything that torch has to see
+    (gradients, transforms, tracing), is that formulation.
     """
+    if group_size == GROUP_SIZE and dtype in (torch.float32, torch.float16):
+        ext = _plain_gpu(packed, scales)
+        if ext is not None:
+            return ext.dequantize(packed, scales, dtype == torch.float16)
+    return dequantize_torch(packed, scales, group_size, dtype)
+
+
+def dequantize_torch(
+    packed: torch.Tensor,
+    scales: torch.Tensor,
+    group_size: int = GROUP_SIZE,
+    dtype: torch.dtype = torch.float32,
+) -> torch.Tensor:
+    """W = q * scale as torch tensor arithmetic, on the inputs' device."""
     q = unpack_to_int(packed).to(dtype)
     m, k = q.shape
     s = scales.to(dtype).reshape(m, k // group_size, 1)

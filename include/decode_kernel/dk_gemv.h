@@ -212,6 +212,12 @@ int dk_w4a16_gemv_paired(const uint32_t* paired, const uint16_t* scales,
 int dk_quantize_pack_f32(const float* w, int M, int K, uint32_t* packed,
                          uint16_t* scales, hipStream_t stream);
 
+/* W = q * scale [M, K] in fp32 (exact), or with fp16 nonzero in fp16 (one
+ * rounding), 16-byte aligned. Replaces dequantize on device tensors
+ * (python/decode_kernel/quantize.py:66-78). */
+int dk_dequantize(const uint32_t* packed, const uint16_t* scales, int M, int K, int fp16,
+                  void* out, hipStream_t stream);
+
 /* STREAM probes. Reference: include/decode_kernel/gemv_w4a16.h:38-43,
  * csrc/gemv_w4a16.cu:593-626. `bytes` must be a multiple of 16.
  * dk_stream_read writes one fp32 partial sum per block into `partials`
