@@ -388,23 +388,33 @@ __global__ __launch_bounds__(WMN * WKN * 64, 2) void gemm_w4(
   }
   gemm_wait<0, true>();
 
-  // The sums go through LDS, 32 batch rows at a time, where the K parts meet
-  // (added in order) and from where rows leave 8 columns to a lane. Columns
-  // are swapped by halves in every other four rows, so that the two halves of
-  // a wave's store take different banks.
+  // The sums go through LDS, as many batch rows at a time as fit, where the K
+  // parts meet (added in order) and from where rows leave 8 columns to a lane.
+  // Columns are swapped by halves in every other four rows, so that the two
+  // halves of a wave's store take different banks. A wave without other K
+  // parts reads only its own, with no barrier.
   float* red = reinterpret_cast<float*>(&lds);
+  constexpr int kAtOnce = WKN > 1 && NBT == 4 ? 2 : 1;  // 32-row b tiles
+  static_assert(kWaves * kAtOnce * 8192 <= sizeof(Lds), "room for the sums");
   constexpr int kPerRow = kRows / 8;  // 8-column pieces of an output row
-  constexpr int kPieces = 32 * kPerRow / WKN;
+  constexpr int kPieces = 32 * kAtOnce * kPerRow / WKN;
   const bool wide = M % 8 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
 #pragma unroll
-  for (int j = 0; j < NBT; ++j) {
-    float* mine = red + wave * 2048 + half * 256 + (r32 ^ (32 * half));
+  for (int j = 0; j < NBT; j += kAtOnce) {
+    float* mine = red + wave * kAtOnce * 2048 + half * 256 + (r32 ^ (32 * half));
+    if (WKN > 1 && j > 0) __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int d = 0; d < kAtOnce; ++d)
 #pragma unroll
-      for (int v = 0; v < 16; ++v)
-        mine[(8 * (v / 4) + v % 4) * 64 + (half ? -32 * i : 32 * i)] = tot[i][j][v];
-    __syncthreads();
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          mine[d * 2048 + (8 * (v / 4) + v % 4) * 64 + (half ? -32 * i : 32 * i)] =
+              tot[i][j + d][v];
+    if constexpr (WKN > 1)
+      __syncthreads();
+    else
+      wave_lds_sync();
 #pragma unroll
     for (int u = 0; u < (kPieces + 63) / 64; ++u) {
       const int piece = kk * kPieces + u * 64 + lane;
@@ -412,12 +422,12 @@ __global__ __launch_bounds__(WMN * WKN * 64, 2) void gemm_w4(
       const int b = b0 + 32 * j + row, m = m0 + 8 * c8;
       const int swap = row & 4;
       if ((kPieces < 64 && lane >= kPieces) || b >= B) continue;
-      const float* from = red + wm * 2048 + row * 64;
+      const float* from = red + wm * kAtOnce * 2048 + row * 64;
       auto sum = [&](int c, float (&out)[8]) {
 #pragma unroll
         for (int q = 0; q < WKN; ++q) {
-          const float4* f =
-              reinterpret_cast<const float4*>(from + q * (WMN * 2048) + 8 * (c ^ swap));
+          const float4* f = reinterpret_cast<const float4*>(from + q * (WMN * kAtOnce * 2048) +
+                                                            8 * (c ^ swap));
           const float part[8] = {f[0].x, f[0].y, f[0].z, f[0].w, f[1].x, f[1].y, f[1].z, f[1].w};
 #pragma unroll
           for (int e = 0; e < 8; ++e) out[e] = q ? out[e] + part[e] : part[e];
@@ -445,7 +455,7 @@ __global__ __launch_bounds__(WMN * WKN * 64, 2) void gemm_w4(
           if (m + e < M) to[e] = f2h(a[e]);
       }
     }
-    __syncthreads();
+    if constexpr (WKN == 1) wave_lds_sync();
   }
 }
 
