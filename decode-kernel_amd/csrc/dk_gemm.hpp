@@ -124,28 +124,33 @@ __device__ __forceinline__ void gemm_wait() {
 }
 
 // A stream is the WMN waves that share x: the same batch rows and groups.
-template <int kWaves, int WMN>
+// kGroups: weights are loaded so many groups ahead.
+template <int kWaves, int WMN, int MT>
 struct GemmLds {
   static constexpr int kStreams = kWaves / WMN;
   static constexpr int kUnit = WMN * 256;  // uint4 of a stream's unit of x
   static constexpr int kRing = 3;          // units staged
   uint4 x[kRing][kStreams * kUnit];
-  uint4 w[kWaves][256];  // a wave's 64 rows of one group
-  uint32_t s[kWaves][2][64];
+  static constexpr int kGroups = MT == 1 ? 2 : 1;
+  uint4 w[kGroups][kWaves][MT * 128];  // a wave's rows of one group
+  uint32_t s[kGroups][kWaves][MT][64];
 };
 
-// WMN waves side by side (64 rows of W each, or 32 of Wg and of Wu) by WKN
-// waves that take every WKN-th group of K; each wave 32 NBT batch rows. x is
+// WMN waves side by side (MT row tiles of 32 each; for gate/up one of Wg and
+// one of Wu) by WKN waves that take every WKN-th group of K; each wave 32 NBT
+// batch rows. With MT = 1, for batches whose grid would leave CUs idle or a
+// step waiting for HBM, the weights are half as many, so two groups of them
+// are staged (5000 x 4224, B = 17: 8.6 us against 11.8 for MT = 2). x is
 // staged in units: with WMN > 1 of 16 WMN batch rows by a group, with WMN = 1,
 // where no other wave reads them and no barrier is needed, of 32 rows by half
 // a group. P units make a group; unit u + 2 is issued during unit u.
-template <int WMN, int WKN, int NBT, bool kGateUp>
+template <int WMN, int WKN, int NBT, int MT, bool kGateUp>
 __global__ __launch_bounds__(WMN * WKN * 64, 2) void gemm_w4(
     const uint4* __restrict__ w0p, const uint16_t* __restrict__ s0p, const uint4* __restrict__ w1p,
     const uint16_t* __restrict__ s1p, const uint4* __restrict__ x4, uint16_t* __restrict__ y, int M,
     int K, int B) {
   constexpr int kWaves = WMN * WKN;
-  using Lds = GemmLds<kWaves, WMN>;
+  using Lds = GemmLds<kWaves, WMN, MT>;
   constexpr bool kShared = WMN > 1;
   constexpr int kHalves = kShared ? 1 : 2;       // units per b tile
   constexpr int kTiles = kShared ? WMN / 2 : 1;  // 32-row b tiles per unit
@@ -153,8 +158,9 @@ __global__ __launch_bounds__(WMN * WKN * 64, 2) void gemm_w4(
   constexpr int P = NBT * kHalves / kTiles;      // units per group
   constexpr int kNx = 4;                         // x loads per wave and unit
   constexpr int kAhead = Lds::kRing - 1;         // units issued ahead
-  constexpr int kNw = 6;                         // weight and scale loads per wave and group
-  constexpr int kRows = kGateUp ? 32 : 64;       // output rows per wave
+  constexpr int kNw = 3 * MT;                    // weight and scale loads per wave and group
+  constexpr int kRows = kGateUp ? 32 : 32 * MT;  // output rows per wave
+  static_assert(MT == 2 || (!kShared && !kGateUp), "one m tile: private x, one matrix");
   static_assert(kAhead <= P && kNx * WMN * kHalves == 8 * kTiles, "load counts");
   using std::integral_constant;
   __shared__ Lds lds;
@@ -204,10 +210,11 @@ __global__ __launch_bounds__(WMN * WKN * 64, 2) void gemm_w4(
     issue_x(r, lds0, integral_constant<int, 2>());
     issue_x(r, lds0, integral_constant<int, 3>());
   };
-  // Weights: load i covers rows 16 i .. + 15 of the wave's 64, lane l the
+  // Weights: load i covers rows 16 i .. + 15 of the wave's, lane l the
   // slot l % 4 of row l / 4, which holds chunk (l % 4) ^ (row / 4 % 4).
-  const uint32_t wl = lds_address(&lds.w[wave][0]);
-  const uint32_t sl = lds_address(&lds.s[wave][0][0]);
+  const uint32_t wl = lds_address(&lds.w[0][wave][0]);
+  const uint32_t sl = lds_address(&lds.s[0][wave][0][0]);
+  constexpr uint32_t kWSlot = kWaves * MT * 2048, kSSlot = kWaves * MT * 256;
   const uint32_t wrow = (uint32_t)K / 2;
   const uint32_t woff = (lane >> 2) * wrow + (((lane & 3) ^ ((lane >> 4) & 3)) << 4);
   const int wleft = __builtin_amdgcn_readfirstlane(min(kRows, M - m0));
@@ -219,26 +226,28 @@ __global__ __launch_bounds__(WMN * WKN * 64, 2) void gemm_w4(
   const char* sg0 = reinterpret_cast<const char*>(s0p) + ((size_t)m0 * G + gfirst) * 2;
   const char* sg1 = reinterpret_cast<const char*>(kGateUp ? s1p : s0p) +
                     ((size_t)(m0 + row1) * G + gfirst) * 2;
-  auto issue_w = [&](auto iv) {  // i < 4: weights, else scales
+  uint32_t wbuf = 0;  // the buffer of the group at hand (two with one m tile)
+  auto issue_w = [&](auto iv) {  // i < 2 MT: weights, else scales
     constexpr int i = decltype(iv)::value;
-    constexpr int t = i < 4 ? i / 2 : i - 4;
-    if constexpr (i < 4) {
+    constexpr int t = i < 2 * MT ? i / 2 : i - 2 * MT;
+    if constexpr (i < 2 * MT) {
       uint32_t wo = woff;
       asm volatile("" : "+v"(wo));
-      dma16<i * 1024>(wl, i % 2 ? wo + 16 * wrow : wo,
+      dma16<i * 1024>(wl + wbuf * kWSlot, i % 2 ? wo + 16 * wrow : wo,
                       gemm_rsrc(t ? wg1 : wg0, (t ? left1 : left0) * wrow));
     } else {
       uint32_t r = threadIdx.x;
       asm volatile("" : "+v"(r));
-      dma2<t * 256>(sl, (r & 31) * (uint32_t)G * 2, gemm_rsrc(t ? sg1 : sg0, (t ? left1 : left0) * (2 * G)));
+      dma2<t * 256>(sl + wbuf * kSSlot, (r & 31) * (uint32_t)G * 2,
+                    gemm_rsrc(t ? sg1 : sg0, (t ? left1 : left0) * (2 * G)));
     }
   };
 
   // tot[i][j]: the sums of the wave's m tile i and b tile j (32 x 32), this
   // lane's column lane % 32 and rows 8 (v / 4) + 4 (lane / 32) + v % 4.
-  f16_t tot[2][NBT];
+  f16_t tot[MT][NBT];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < MT; ++i)
 #pragma unroll
     for (int j = 0; j < NBT; ++j)
 #pragma unroll
@@ -259,28 +268,48 @@ __global__ __launch_bounds__(WMN * WKN * 64, 2) void gemm_w4(
   // Words t = 4 n .. 4 n + 3 of the wave's tile i.
   auto read_words = [&](uint32_t (&a)[8], int i, int n) {
     if constexpr (kHalves == 1) {
-      const u32x4_t v = *(lds_u4_ptr)(uintptr_t)((wread ^ (16u * n)) + i * 2048);
+      const u32x4_t v =
+          *(lds_u4_ptr)(uintptr_t)((wread ^ (16u * n)) + wbuf * kWSlot + i * 2048);
       a[4 * n] = v.x, a[4 * n + 1] = v.y, a[4 * n + 2] = v.z, a[4 * n + 3] = v.w;
     } else {
 #pragma unroll
       for (int t = 4 * n; t < 4 * n + 4; ++t)
-        a[t] = *(lds_u32_ptr)(uintptr_t)((wread ^ (16u * (t / 2))) + i * 2048 + t % 2 * 8);
+        a[t] = *(lds_u32_ptr)(uintptr_t)((wread ^ (16u * (t / 2))) + wbuf * kWSlot + i * 2048 +
+                                         t % 2 * 8);
     }
   };
 
-  issue_w(integral_constant<int, 0>());
-  issue_w(integral_constant<int, 1>());
-  issue_w(integral_constant<int, 2>());
-  issue_w(integral_constant<int, 3>());
-  issue_w(integral_constant<int, 4>());
-  issue_w(integral_constant<int, 5>());
+  // Past a row's end the last group's loads are repeated and not used.
+  auto next_w = [&](bool more) {
+    wg0 += more ? WKN * 64 : 0;
+    wg1 += more ? WKN * 64 : 0;
+    sg0 += more ? WKN * 2 : 0;
+    sg1 += more ? WKN * 2 : 0;
+  };
+  auto issue_w_all = [&] {
+    issue_w(integral_constant<int, 0>());
+    issue_w(integral_constant<int, 1>());
+    issue_w(integral_constant<int, 2>());
+    if constexpr (MT == 2) {
+      issue_w(integral_constant<int, 3>());
+      issue_w(integral_constant<int, 4>());
+      issue_w(integral_constant<int, 5>());
+    }
+  };
+  issue_w_all();
+  if constexpr (Lds::kGroups == 2) {
+    next_w(1 < its);
+    wbuf = 1;
+    issue_w_all();
+    wbuf = 0;
+  }
 #pragma unroll
   for (int u = 0; u < kAhead; ++u) issue_x_all(x_rsrc(xg, u), xl + u * kSlot);
   for (int d = 0; d < lag; ++d) asm volatile("s_barrier" ::: "memory");
   // A tile's sums of the group wait in acc for the next tile's loads: they
   // are scaled and added to tot while those arrive.
-  f16_t acc[2] = {};
-  float sc[2] = {0.0f, 0.0f};
+  f16_t acc[MT] = {};
+  float sc[MT] = {};
   auto add_scaled = [&](f16_t& sum, int i) {
 #pragma unroll
     for (int v = 0; v < 16; ++v) sum[v] = __builtin_fmaf(acc[i][v], sc[i], sum[v]);
@@ -288,15 +317,10 @@ __global__ __launch_bounds__(WMN * WKN * 64, 2) void gemm_w4(
   };
   uint32_t slot = 0;  // byte offset of the unit's slot
   for (int it = 0; it < its; ++it) {
-    // Past the end the last group's loads are repeated and not used.
-    const bool more = it + 1 < its;
-    wg0 += more ? WKN * 64 : 0;
-    wg1 += more ? WKN * 64 : 0;
-    sg0 += more ? WKN * 2 : 0;
-    sg1 += more ? WKN * 2 : 0;
-    const char* xnext = xg + (more ? WKN * 256 : 0);
-    h8_t wq[2][8];
-    uint32_t a[2][8];
+    next_w(it + Lds::kGroups < its);
+    const char* xnext = xg + (it + 1 < its ? WKN * 256 : 0);
+    h8_t wq[MT][8];
+    uint32_t a[MT][8];
 #pragma unroll
     for (int p = 0; p < P; ++p) {
       // In flight beyond this unit's x: that of the next units, and the next
@@ -315,26 +339,28 @@ __global__ __launch_bounds__(WMN * WKN * 64, 2) void gemm_w4(
       h8_t xf[kRing];
 #pragma unroll
       for (int s = 0; s < kRing - 1; ++s) xf[s] = frag(s);
-      float next_sc[2];
+      float next_sc[MT];
       if (p == 0) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
+        for (int i = 0; i < MT; ++i) {
           read_words(a[i], i, 0);
           uint32_t r = threadIdx.x;
           asm volatile("" : "+v"(r));
-          next_sc[i] = h2f((uint16_t) * (lds_u32_ptr)(uintptr_t)(sl + i * 256 + (r & 31) * 4));
+          next_sc[i] = h2f((uint16_t) * (lds_u32_ptr)(uintptr_t)(sl + wbuf * kSSlot + i * 256 +
+                                                                 (r & 31) * 4));
         }
       }
       if (p % kHalves == 0) {
         const int prev = ((p + P - 1) % P / kHalves + 1) * kTiles - 1;
-        add_scaled(tot[0][prev], 0);
-        add_scaled(tot[1][prev], 1);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) add_scaled(tot[i][prev], i);
       }
       if (p == 0) {
-        wq[0][0] = unpack_word_natural(a[0][0]);
-        wq[1][0] = unpack_word_natural(a[1][0]);
-        sc[0] = next_sc[0];
-        sc[1] = next_sc[1];
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+          wq[i][0] = unpack_word_natural(a[i][0]);
+          sc[i] = next_sc[i];
+        }
       }
       const uint32_t ahead = xl + (slot == 0 ? kAhead * kSlot : slot - kSlot);
       const u32x4_t xr = x_rsrc(p + kAhead < P ? xg : xnext, (p + kAhead) % P);
@@ -344,7 +370,7 @@ __global__ __launch_bounds__(WMN * WKN * 64, 2) void gemm_w4(
         const int t = s % kSteps + p % kHalves * kSteps;  // of the tile's eight
         if (s + kRing - 1 < kSteps * kTiles) xf[(s + kRing - 1) % kRing] = frag(s + kRing - 1);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
+        for (int i = 0; i < MT; ++i) {
           if (t == 0 && s > 0) add_scaled(tot[i][p * kTiles + s / kSteps - 1], i);
           const f16_t zero = {};
           acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[s % kRing], wq[i][t],
@@ -353,23 +379,28 @@ __global__ __launch_bounds__(WMN * WKN * 64, 2) void gemm_w4(
           // The loads and the rest of the decode go out between the MFMAs.
           if (p < kHalves && s < kSteps && t < 7) wq[i][t + 1] = unpack_word_natural(a[i][t + 1]);
           if (p == 0 && s == 0) read_words(a[i], i, 1);
-          const int n = s * 2 + i;
-          constexpr int kW = kHalves == 1 ? 6 : 2;  // slots of the first loads
-          const int kX = kHalves == 1 ? 12 : p == 0 ? 4 : 1;
+          // Slots of the first loads; two loads to a slot with one m tile.
+          const int n = (s * MT + i) * (3 - MT);
+          constexpr int kW = kHalves == 1 ? 6 : 2;
+          const int kX = kHalves == 1 ? 12 : p == 0 ? 4 : MT == 2 ? 1 : 0;
+#define DK_AT(first, i) (n <= (first) + (i) && (first) + (i) < n + 3 - MT)
           if (p == 0) {
-            // The group's words have left the buffer that the next group's take.
+            // The group's words have left the buffer that these loads take.
             if (n == kW) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            if (n == kW) issue_w(integral_constant<int, 0>());
-            if (n == kW + 1) issue_w(integral_constant<int, 1>());
-            if (n == kW + 2) issue_w(integral_constant<int, 2>());
-            if (n == kW + 3) issue_w(integral_constant<int, 3>());
-            if (n == kW + 4) issue_w(integral_constant<int, 4>());
-            if (n == kW + 5) issue_w(integral_constant<int, 5>());
+            if (DK_AT(kW, 0)) issue_w(integral_constant<int, 0>());
+            if (DK_AT(kW, 1)) issue_w(integral_constant<int, 1>());
+            if (DK_AT(kW, 2)) issue_w(integral_constant<int, 2>());
+            if constexpr (MT == 2) {
+              if (DK_AT(kW, 3)) issue_w(integral_constant<int, 3>());
+              if (DK_AT(kW, 4)) issue_w(integral_constant<int, 4>());
+              if (DK_AT(kW, 5)) issue_w(integral_constant<int, 5>());
+            }
           }
-          if (n == kX) issue_x(xr, ahead, integral_constant<int, 0>());
-          if (n == kX + 1) issue_x(xr, ahead, integral_constant<int, 1>());
-          if (n == kX + 2) issue_x(xr, ahead, integral_constant<int, 2>());
-          if (n == kX + 3) issue_x(xr, ahead, integral_constant<int, 3>());
+          if (DK_AT(kX, 0)) issue_x(xr, ahead, integral_constant<int, 0>());
+          if (DK_AT(kX, 1)) issue_x(xr, ahead, integral_constant<int, 1>());
+          if (DK_AT(kX, 2)) issue_x(xr, ahead, integral_constant<int, 2>());
+          if (DK_AT(kX, 3)) issue_x(xr, ahead, integral_constant<int, 3>());
+#undef DK_AT
           __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -377,9 +408,10 @@ __global__ __launch_bounds__(WMN * WKN * 64, 2) void gemm_w4(
       slot = slot == kAhead * kSlot ? 0 : slot + kSlot;
     }
     xg = xnext;
+    if constexpr (Lds::kGroups == 2) wbuf ^= 1;
   }
-  add_scaled(tot[0][NBT - 1], 0);
-  add_scaled(tot[1][NBT - 1], 1);
+#pragma unroll
+  for (int i = 0; i < MT; ++i) add_scaled(tot[i][NBT - 1], i);
   if constexpr (kShared) {
     // Every wave meets the same barriers: those of a group it has not, and the
     // half group by which the other waves lag.
@@ -390,27 +422,29 @@ __global__ __launch_bounds__(WMN * WKN * 64, 2) void gemm_w4(
 
   // The sums go through LDS, as many batch rows at a time as fit, where the K
   // parts meet (added in order) and from where rows leave 8 columns to a lane.
-  // Columns are swapped by halves in every other four rows, so that the two
-  // halves of a wave's store take different banks. A wave without other K
+  // In every other four rows the halves of the columns (with one m tile, the
+  // rows of a pair) are swapped, so that the two halves of a wave's store take
+  // different banks. A wave without other K
   // parts reads only its own, with no barrier.
   float* red = reinterpret_cast<float*>(&lds);
   constexpr int kAtOnce = WKN > 1 && NBT == 4 ? 2 : 1;  // 32-row b tiles
-  static_assert(kWaves * kAtOnce * 8192 <= sizeof(Lds), "room for the sums");
+  constexpr int kCols = 32 * MT, kTile = 32 * kCols;
+  static_assert(kWaves * kAtOnce * kTile * 4 <= sizeof(Lds), "room for the sums");
   constexpr int kPerRow = kRows / 8;  // 8-column pieces of an output row
   constexpr int kPieces = 32 * kAtOnce * kPerRow / WKN;
   const bool wide = M % 8 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
 #pragma unroll
   for (int j = 0; j < NBT; j += kAtOnce) {
-    float* mine = red + wave * kAtOnce * 2048 + half * 256 + (r32 ^ (32 * half));
+    float* mine = red + wave * kAtOnce * kTile + r32 + half * (4 * kCols);
+    float* const put[2] = {mine + half * 32, mine - half * 32 + (MT == 2 ? 32 : 0)};
     if (WKN > 1 && j > 0) __syncthreads();
 #pragma unroll
     for (int d = 0; d < kAtOnce; ++d)
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int v = 0; v < 16; ++v)
-          mine[d * 2048 + (8 * (v / 4) + v % 4) * 64 + (half ? -32 * i : 32 * i)] =
-              tot[i][j + d][v];
+          put[MT == 2 ? i : v % 2][d * kTile + (8 * (v / 4) + v % 4) * kCols] = tot[i][j + d][v];
     if constexpr (WKN > 1)
       __syncthreads();
     else
@@ -421,13 +455,14 @@ __global__ __launch_bounds__(WMN * WKN * 64, 2) void gemm_w4(
       const int row = piece / kPerRow, c8 = piece % kPerRow;
       const int b = b0 + 32 * j + row, m = m0 + 8 * c8;
       const int swap = row & 4;
+      const int at = MT == 2 ? row * kCols : (row ^ (swap >> 2)) * kCols;
       if ((kPieces < 64 && lane >= kPieces) || b >= B) continue;
-      const float* from = red + wm * kAtOnce * 2048 + row * 64;
+      const float* from = red + wm * kAtOnce * kTile + at;
       auto sum = [&](int c, float (&out)[8]) {
 #pragma unroll
         for (int q = 0; q < WKN; ++q) {
-          const float4* f = reinterpret_cast<const float4*>(from + q * (WMN * kAtOnce * 2048) +
-                                                            8 * (c ^ swap));
+          const float4* f = reinterpret_cast<const float4*>(from + q * (WMN * kAtOnce * kTile) +
+                                                            8 * (MT == 2 ? c ^ swap : c));
           const float part[8] = {f[0].x, f[0].y, f[0].z, f[0].w, f[1].x, f[1].y, f[1].z, f[1].w};
 #pragma unroll
           for (int e = 0; e < 8; ++e) out[e] = q ? out[e] + part[e] : part[e];

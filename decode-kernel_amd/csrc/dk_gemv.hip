@@ -439,42 +439,44 @@ int launch_v5(const Launch& L, const uint4* p, const uint16_t* s, const uint4* x
 }
 #undef DK_BATCH
 
-// The many-batch kernel (gemm_w4): WMN x WKN waves, 32 NBT batch rows per
-// workgroup; wmn = 0: not this kernel.
+// The many-batch kernel (gemm_w4): WMN x WKN waves of MT row tiles (32 rows
+// each), 32 NBT batch rows per workgroup; wmn = 0: not this kernel.
 struct GemmShape {
-  int wmn = 0, wkn = 0, nbt = 0;
+  int wmn = 0, wkn = 0, nbt = 0, mt = 0;
 };
 
 long long ceil_div(long long a, long long b) { return (a + b - 1) / b; }
 
-// The shape with the least estimated time for M rows, `unit` of them per wave
-// (64; 32 of each matrix for gate/up). A workgroup takes fixed + step us per
-// step (one group per K part); eight-wave workgroups run one to a CU, in
+// The shape with the least estimated time. A workgroup takes fixed + step us
+// per step (one group per K part); eight-wave workgroups run one to a CU, in
 // rounds of 256; four-wave ones two to a CU when there are more than 256, a
-// pair then taking `pair` us per step. Fitted to the seven shapes' times over
-// 15 (M, K) from 512 x 4096 to 28672 x 8192 and six of gate/up, at 15 batches
-// from 17 to 1000: the choice is 0.1% from the best shape on average and 5% at
-// worst. What decides is the number of workgroups: few take many K parts and
-// few batch rows each, many decode each weight for 128 batch rows and leave
-// the CU to two workgroups (us, the choice first; 4096 x 4096, B = 64 10.8 for
-// <1, 8, 1>, 13.9 for <1, 8, 2>, 19.7 for <2, 4, 2>; B = 1000 38.2 for
-// <2, 4, 4>, 42.3 for <1, 4, 4>, 49.6 for <1, 8, 4>, 64.4 for <4, 1, 4>; 28672
-// x 8192, B = 2048 820 for <4, 1, 4>, 972 for <2, 4, 4>).
-GemmShape gemm_best(int M, int K, int B, int unit) {
+// pair then taking `pair` us per step. Fitted to the shapes' times over 18
+// (M, K) from 512 x 4096 to 28672 x 8192 and six of gate/up, at batches from
+// 17 to 1000: the choice is 0.2% from the best shape on average and 5% at
+// worst. What decides is the number of workgroups: few take many K parts, few
+// batch rows and one row tile each, many decode each weight for 128 batch rows
+// and leave the CU to two workgroups (us, the choice first; MT = 2 but where
+// noted; 5000 x 4224, B = 17 8.6 for <1, 8, 1, MT = 1>, 11.8 for <1, 8, 1>;
+// 4096 x 4096, B = 1000 38.2 for <2, 4, 4>, 42.3 for <1, 4, 4>, 49.6 for
+// <1, 8, 4>, 64.4 for <4, 1, 4>; 28672 x 8192, B = 2048 820 for <4, 1, 4>, 972
+// for <2, 4, 4>). Gate/up has a row tile of each matrix: MT = 2 only.
+GemmShape gemm_best(int M, int K, int B, bool gate_up) {
   struct Cand {
-    int wmn, wkn, nbt;
+    int wmn, wkn, nbt, mt;
     double fixed, step, pair;
   };
   constexpr Cand kCands[] = {
-      {1, 8, 1, 3.8, 2.0, 0.0}, {1, 8, 2, 4.0, 3.0, 0.0}, {2, 4, 2, 4.3, 2.36, 0.0},
-      {1, 8, 4, 5.4, 4.6, 0.0}, {2, 4, 4, 6.2, 3.74, 0.0}, {1, 4, 4, 3.7, 2.95, 4.1},
-      {4, 1, 4, 3.0, 2.1, 3.47},
+      {1, 8, 1, 1, 3.8, 1.1, 0.0},  {1, 8, 2, 1, 4.0, 1.62, 0.0}, {1, 8, 1, 2, 4.0, 1.62, 0.0},
+      {1, 8, 2, 2, 4.0, 3.0, 0.0},  {2, 4, 2, 2, 4.3, 2.36, 0.0}, {1, 8, 4, 2, 5.4, 4.6, 0.0},
+      {2, 4, 4, 2, 6.2, 3.62, 0.0}, {1, 4, 4, 2, 3.7, 2.95, 4.1}, {4, 1, 4, 2, 3.0, 2.1, 3.47},
   };
   const int G = K / DK_GROUP_SIZE;
   GemmShape best;
   double best_us = 0.0;
   for (const Cand& c : kCands) {
-    const long long n = ceil_div(M, unit * c.wmn) * ceil_div(B, 32 * c.nbt);
+    if (gate_up && c.mt == 1) continue;
+    const int rows = (gate_up ? 32 : 32 * c.mt) * c.wmn;
+    const long long n = ceil_div(M, rows) * ceil_div(B, 32 * c.nbt);
     if (n > 0x7fffffffLL) continue;
     const double steps = (double)ceil_div(G, c.wkn);
     double us;
@@ -486,7 +488,7 @@ GemmShape gemm_best(int M, int K, int B, int unit) {
            (rest ? c.fixed + steps * (rest > 256 ? c.pair : c.step) : 0.0);
     }
     if (best.wmn == 0 || us < best_us) {
-      best = {c.wmn, c.wkn, c.nbt};
+      best = {c.wmn, c.wkn, c.nbt, c.mt};
       best_us = us;
     }
   }
@@ -494,43 +496,57 @@ GemmShape gemm_best(int M, int K, int B, int unit) {
 }
 
 // Where gemm_w4 takes the weight-reuse path's batches (`pairs`: the scales
-// load in pairs) and gate/up's: above 16 batch rows, where its workgroups,
-// 64 rows by 32-128 batch rows each, fill half the chip. Its 32-bit offsets
-// take K up to 2^21. Against the 16-row tiles (us, gemm_w4 first):
-//   pairs:  M = K = 4096, B = 64 10.8 (9.3), 96 13.8 (14.1), 192 14.4 (21.7);
-//           M = 2048, K = 11008, B = 128 29.8 (18.7), 256 30.8 (31.1), 512 47.7 (51.4);
-//           M = 1024, K = 8192, B = 512 24 (25.7), 1000 37.9 (41.2);
-//           M = 8192, K = 28672, B = 32 53.4 (46.5), 48 51.5 (69.2);
-//           M = 11008, K = 4096, B = 17 11.0 (14.4);
+// load in pairs) and gate/up's: above 16 batch rows, where its tiles come near
+// to one per CU. Its 32-bit offsets take K up to 2^21. Against the 16-row
+// tiles (us over cold weights, gemm_w4 first):
+//   pairs, above 32 batch rows: over 256 tiles of 32 x 32, for a launch of
+//           them takes as long as one of half as many:
+//           M = 1024, K = 8192, B = 256 19.5 (14.0); K = 4096, B = 288 10.8 (12.6);
+//           M = K = 4096, B = 64 9.2 (8.6), 96 11.6 (13.1), 256 16.2 (20.5);
+//           M = K = 8192, B = 48 21.0 (23.9), 128 28.8 (37.3), 256 44.0 (66.1);
+//           M = 5632, K = 28672, B = 33 56.8 (65.6), 64 66.7 (66.8);
 //           rows of up to 1024 weights stay (M = 4096, K = 1024, B = 64 5.3
-//           (4.7), 128 6.7 (6.7), 256 6.9 (8.7))
-//   no pairs (the 16-row tiles then cost the same for every 16 batch rows):
-//           M = 4096, K = 4224, B = 32 10.7 (7.7), 64 11.1 (13.4);
-//           M = 512, K = 4224, B = 256 13.1 (10.4), 512 14.6 (20.0)
+//           (4.7), 128 6.7 (6.7), 256 6.9 (8.7));
+//   pairs, 17 to 32 batch rows: over 8192 rows, B K up to 3 2^16, for each
+//           workgroup stages x by itself (the 16-row tiles read it through L1):
+//           M = 8448, K = 4096, B = 17 11.9 (14.8), 32 13.2 (15.4);
+//           M = 28672, K = 8192, B = 17 43.1 (46.1);  M = 9216, B = 32 24.5 (23.3);
+//           M = 10240, K = 28672, B = 17 68.3 (65.5), 32 77.5 (68.1)
+//   no pairs (the 16-row tiles are slower there): over 512 tiles of 16 x 16, above 32 batch rows
+//           384 from 1025 rows on:
+//           M = 5000, K = 4224, B = 17 8.6 (11.7), 64 12.0 (18.6);
+//           M = 3584, K = 10880, B = 17 16.7 (14.1); M = 4608 17.1 (21.4);
+//           M = 1536, K = 10880, B = 33 15.6 (13.6), 64 18.0 (19.4);
+//           M = 2048, K = 1152, B = 33 4.8 (5.9); M = 1024, K = 10880, B = 128 17.2 (16.8)
 //   gate/up, likewise:
 //           I = 2048, H = 4096, B = 64 11.0 (10.2), 128 15.7 (17.7);
 //           I = 3584, H = 8192, B = 32 18.3 (19.9), 48 18.5 (28.1);
 //           I = 11008, H = 4096, B = 16 20.5 (16.0), 17 20.3 (23.6)
 GemmShape gemm_shape(int M, int K, int B, bool pairs) {
   if (B <= 16 || K > (1 << 21)) return {};
-  const bool take =
-      pairs ? K > 1024 && (M > 8192 || (B > 32 && ceil_div(M, 64) * ceil_div(B, 64) >= 128))
-            : ceil_div(M, 16) * ceil_div(B, 16) > 512;
-  return take ? gemm_best(M, K, B, 64) : GemmShape{};
+  bool take;
+  if (pairs && B <= 32) {
+    take = K > 1024 && M > 8192 && B * K <= 3 << 16;
+  } else if (pairs) {
+    take = K > 1024 && ceil_div(M, 32) * ceil_div(B, 32) > 256;
+  } else {
+    take = ceil_div(M, 16) * ceil_div(B, 16) >= (B > 32 && M > 1024 ? 384 : 513);
+  }
+  return take ? gemm_best(M, K, B, false) : GemmShape{};
 }
 
 GemmShape gate_up_gemm_shape(int I, int H, int B) {
   if (B <= 16 || H > (1 << 21) || ceil_div(I, 16) * ceil_div(B, 16) <= 512) return {};
-  return gemm_best(I, H, B, 32);
+  return gemm_best(I, H, B, true);
 }
 
-template <int WMN, int WKN, int NBT, bool kGateUp>
+template <int WMN, int WKN, int NBT, int MT, bool kGateUp>
 int launch_gemm_t(const Launch& L, const char* what, const uint4* w0, const uint16_t* s0,
                   const uint4* w1, const uint16_t* s1, const uint4* x, uint16_t* y, int M, int K,
                   int B) {
-  const long long n = ceil_div(M, (kGateUp ? 32 : 64) * WMN) * ceil_div(B, 32 * NBT);
-  return L(what, dk::gemm_w4<WMN, WKN, NBT, kGateUp>, dim3((unsigned)n), dim3(WMN * WKN * 64), 0,
-           w0, s0, w1, s1, x, y, M, K, B);
+  const long long n = ceil_div(M, (kGateUp ? 32 : 32 * MT) * WMN) * ceil_div(B, 32 * NBT);
+  return L(what, dk::gemm_w4<WMN, WKN, NBT, MT, kGateUp>, dim3((unsigned)n), dim3(WMN * WKN * 64),
+           0, w0, s0, w1, s1, x, y, M, K, B);
 }
 
 template <bool kGateUp>
@@ -538,14 +554,17 @@ int launch_gemm(const Launch& L, const GemmShape& g, const uint4* w0, const uint
                 const uint4* w1, const uint16_t* s1, const uint4* x, uint16_t* y, int M, int K,
                 int B) {
   const char* what = kGateUp ? "gate/up launch" : "reuse launch";
-#define DK_GEMM(m, k, n)                            \
-  if (g.wmn == m && g.wkn == k && g.nbt == n)       \
-    return launch_gemm_t<m, k, n, kGateUp>(L, what, w0, s0, w1, s1, x, y, M, K, B);
-  DK_GEMM(1, 8, 1) DK_GEMM(1, 8, 2) DK_GEMM(2, 4, 2) DK_GEMM(1, 8, 4) DK_GEMM(2, 4, 4)
-  DK_GEMM(1, 4, 4) DK_GEMM(4, 1, 4)
+#define DK_GEMM(m, k, n, t)                                         \
+  if (g.wmn == m && g.wkn == k && g.nbt == n && g.mt == t)          \
+    return launch_gemm_t<m, k, n, t, kGateUp>(L, what, w0, s0, w1, s1, x, y, M, K, B);
+  if constexpr (!kGateUp) {
+    DK_GEMM(1, 8, 1, 1) DK_GEMM(1, 8, 2, 1)
+  }
+  DK_GEMM(1, 8, 1, 2) DK_GEMM(1, 8, 2, 2) DK_GEMM(2, 4, 2, 2) DK_GEMM(1, 8, 4, 2)
+  DK_GEMM(2, 4, 4, 2) DK_GEMM(1, 4, 4, 2) DK_GEMM(4, 1, 4, 2)
 #undef DK_GEMM
-  return fail(DK_ERR_UNSUPPORTED, "internal: no kernel for %d x %d waves, %d batch tiles", g.wmn,
-              g.wkn, g.nbt);
+  return fail(DK_ERR_UNSUPPORTED, "internal: no kernel for %d x %d waves, %d x %d tiles", g.wmn,
+              g.wkn, g.nbt, g.mt);
 }
 
 // Batches that the MFMA tiles take on the fused gate/up step. Tiles against

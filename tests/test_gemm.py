@@ -27,20 +27,32 @@ def lib():
 
 
 @pytest.mark.parametrize("m,k,b,kernel,blocks", [
-    (4096, 4096, 64, "gemv_reuse_pfb<4, 2, 2>", None),   # 64 x 1 tiles of 64 x 64: below 128
-    (4096, 4096, 65, "gemm_w4<1, 8, 1, false>", 192),
-    (4096, 4096, 129, "gemm_w4<1, 8, 2, false>", 192),
-    (4096, 4096, 1000, "gemm_w4<2, 4, 4, false>", 256),
-    (8192, 8192, 32, "gemv_reuse_pf", None),             # pairs, up to 8192 rows: above 32 rows
-    (8192, 8192, 33, "gemm_w4<1, 8, 1, false>", 256),
-    (8193, 8192, 16, "gemv_reuse", None),
-    (8193, 8192, 17, "gemm_w4<1, 8, 1, false>", 129),
-    (28672, 8192, 2048, "gemm_w4<4, 1, 4, false>", 1792),
-    (4096, 4224, 32, "gemv_reuse_lds<", None),           # no pairs: 256 x 2 tiles of 16 x 16
-    (4096, 4224, 33, "gemm_w4<1, 8, 1, false>", 128),
-    (5000, 4224, 20, "gemm_w4<1, 8, 1, false>", 79),
+    # Scales in pairs, rows of over 1024 weights: over 256 tiles of 32 x 32;
+    # over 8192 rows and up to 3 2^16 activations up to 32 batch rows.
+    (8192, 8192, 17, "gemv_reuse", None),
+    (8193, 8192, 17, "gemm_w4<1, 8, 1, 2, false>", 129),
+    (8193, 6144, 32, "gemm_w4<1, 8, 1, 2, false>", 129),
+    (8193, 6400, 32, "gemv_reuse", None),
+    (12288, 28672, 17, "gemv_reuse", None),
+    (4096, 4096, 64, "gemv_reuse", None),
+    (4096, 4096, 65, "gemm_w4<1, 8, 2, 1, false>", 256),
+    (4097, 4096, 33, "gemm_w4<1, 8, 2, 1, false>", 129),
+    (4096, 4096, 129, "gemm_w4<1, 8, 2, 2, false>", 192),
+    (4096, 4096, 1000, "gemm_w4<2, 4, 4, 2, false>", 256),
+    (1024, 8192, 256, "gemv_reuse", None),
+    (1024, 8192, 257, "gemm_w4<1, 8, 2, 1, false>", 160),
+    (28672, 8192, 2048, "gemm_w4<4, 1, 4, 2, false>", 1792),
+    (4096, 1024, 1000, "gemv_reuse_pfb<", None),
+    # Odd group counts: over 512 tiles of 16 x 16, 384 from 1025 rows on above
+    # 32 batch rows.
+    (4096, 4224, 32, "gemv_reuse_lds<", None),
+    (4097, 4224, 32, "gemm_w4<1, 8, 1, 1, false>", 129),
+    (2032, 4224, 33, "gemv_reuse", None),
+    (2033, 4224, 33, "gemm_w4<1, 8, 1, 1, false>", 128),
+    (1024, 4224, 128, "gemv_reuse", None),
+    (1024, 4224, 129, "gemm_w4<1, 8, 1, 1, false>", 160),
+    (5000, 4224, 20, "gemm_w4<1, 8, 1, 1, false>", 157),
     (256, 1024, 300, "gemv_reuse", None),
-    (4096, 1024, 1000, "gemv_reuse_pfb<", None),         # pairs: rows of over 1024 weights
     (1024, 28672, 33, "gemv_reuse_pf<", None),
     (4096, 1 << 21, 65, "gemm_w4<", None),
     (4096, (1 << 21) + 256, 65, "gemv_reuse_pfb<", None),  # beyond the 32-bit offsets
@@ -55,10 +67,10 @@ def test_linear_routes(lib, m, k, b, kernel, blocks):
 
 @pytest.mark.parametrize("i,h,b,kernel", [
     (11008, 4096, 16, "gate_up_silu_tiles_lds"),
-    (11008, 4096, 17, "gemm_w4<2, 4, 2, true>"),
+    (11008, 4096, 17, "gemm_w4<1, 8, 1, 2, true>"),
     (2048, 4096, 64, "gate_up_silu_tiles_lds"),  # 128 x 4 tiles
-    (2048, 4096, 65, "gemm_w4<1, 8, 1, true>"),
-    (11008, 4096, 1000, "gemm_w4<4, 1, 4, true>"),
+    (2048, 4096, 65, "gemm_w4<1, 8, 1, 2, true>"),
+    (11008, 4096, 1000, "gemm_w4<4, 1, 4, 2, true>"),
     (512, 4096, 20, "gate_up_silu_"),
 ])
 def test_gate_up_routes(lib, i, h, b, kernel):
@@ -100,12 +112,16 @@ def _check(y: torch.Tensor, ref: torch.Tensor, label: str):
 
 
 LINEAR = [
-    ((4161, 384, 17), "<1, 8, 1,"), ((2049, 640, 128), "<1, 8, 1,"), ((8192, 4224, 31), "<1, 8, 1,"),
-    ((8193, 640, 33), "<1, 8, 2,"), ((2113, 1280, 257), "<1, 8, 2,"), ((5000, 4224, 129), "<1, 8, 2,"),
-    ((16392, 1280, 17), "<2, 4, 2,"), ((16385, 640, 64), "<2, 4, 2,"),
-    ((2040, 11136, 640), "<1, 8, 4,"), ((11008, 4224, 129), "<2, 4, 4,"), ((5000, 4224, 520), "<2, 4, 4,"),
-    ((8321, 384, 33), "<1, 4, 4,"), ((2049, 640, 1030), "<1, 4, 4,"),
-    ((4100, 128, 31), "<4, 1, 4,"), ((513, 128, 250), "<4, 1, 4,"), ((16392, 128, 129), "<4, 1, 4,"),
+    ((4161, 384, 17), "<1, 8, 1, 1,"), ((8191, 4224, 31), "<1, 8, 1, 1,"), ((513, 128, 250), "<1, 8, 1, 1,"),
+    ((5000, 4224, 24), "<1, 8, 1, 1,"), ((4095, 2176, 33), "<1, 8, 1, 1,"),
+    ((2049, 640, 128), "<1, 8, 2, 1,"), ((4090, 4224, 65), "<1, 8, 2, 1,"),
+    ((8193, 1280, 17), "<1, 8, 1, 2,"), ((5000, 1152, 80), "<1, 8, 1, 2,"), ((8193, 640, 33), "<1, 8, 2, 2,"),
+    ((5000, 4224, 129), "<1, 8, 2, 2,"),
+    ((16385, 640, 64), "<2, 4, 2, 2,"), ((4100, 4224, 300), "<2, 4, 2, 2,"),
+    ((2040, 11136, 640), "<1, 8, 4, 2,"), ((11008, 4224, 129), "<2, 4, 4, 2,"),
+    ((5000, 4224, 520), "<2, 4, 4, 2,"),
+    ((8321, 384, 33), "<1, 4, 4, 2,"), ((2049, 640, 1030), "<1, 4, 4, 2,"),
+    ((16392, 128, 129), "<4, 1, 4, 2,"), ((2053, 128, 1000), "<4, 1, 4, 2,"),
 ]
 
 
@@ -170,10 +186,10 @@ def test_linear_least_alignment(lib, shape):
 
 
 GATE_UP = [
-    ((4100, 256, 17), "<1, 8, 1,"), ((1000, 384, 250), "<1, 8, 1,"), ((4100, 640, 33), "<1, 8, 2,"),
-    ((2049, 640, 128), "<1, 8, 2,"), ((8193, 384, 17), "<2, 4, 2,"), ((8193, 4224, 65), "<2, 4, 4,"),
-    ((4100, 256, 33), "<1, 4, 4,"), ((3000, 384, 250), "<1, 4, 4,"), ((4100, 128, 17), "<4, 1, 4,"),
-    ((1000, 128, 513), "<4, 1, 4,"), ((2049, 128, 129), "<4, 1, 4,"), ((5888, 13184, 70), "<1, 8, 4,"),
+    ((4100, 256, 17), "<1, 8, 1, 2,"), ((1000, 384, 250), "<1, 8, 1, 2,"), ((4100, 640, 33), "<1, 8, 2, 2,"),
+    ((2049, 640, 128), "<1, 8, 2, 2,"), ((8193, 384, 17), "<2, 4, 2, 2,"), ((8193, 4224, 65), "<2, 4, 4, 2,"),
+    ((4100, 256, 33), "<1, 4, 4, 2,"), ((3000, 384, 250), "<1, 4, 4, 2,"), ((4100, 128, 17), "<4, 1, 4, 2,"),
+    ((1000, 128, 513), "<4, 1, 4, 2,"), ((2049, 128, 129), "<4, 1, 4, 2,"), ((5888, 13184, 70), "<1, 8, 4, 2,"),
 ]
 
 
