@@ -60,17 +60,17 @@ void check_gemv_inputs(const torch::Tensor& packed, const torch::Tensor& scales,
 
 }  // namespace
 
-torch::Tensor gemv_common(torch::Tensor packed, torch::Tensor scales, torch::Tensor x, int version,
-                          int split_k, bool reuse_weights, int warps_per_row);
+torch::Tensor gemv_common(const torch::Tensor& packed, const torch::Tensor& scales,
+                          const torch::Tensor& x, int version, int split_k, bool reuse_weights, int warps_per_row);
 
 // Reference: csrc/bindings.cpp:37-78.
-torch::Tensor w4a16_gemv(torch::Tensor packed, torch::Tensor scales, torch::Tensor x, int version,
-                         int split_k, bool reuse_weights, int warps_per_row) {
+torch::Tensor w4a16_gemv(const torch::Tensor& packed, const torch::Tensor& scales,
+                         const torch::Tensor& x, int version, int split_k, bool reuse_weights, int warps_per_row) {
   return gemv_common(packed, scales, x, version, split_k, reuse_weights, warps_per_row);
 }
 
-torch::Tensor gemv_common(torch::Tensor packed, torch::Tensor scales, torch::Tensor x, int version,
-                          int split_k, bool reuse_weights, int warps_per_row) {
+torch::Tensor gemv_common(const torch::Tensor& packed, const torch::Tensor& scales,
+                          const torch::Tensor& x, int version, int split_k, bool reuse_weights, int warps_per_row) {
   check_gemv_inputs(packed, scales, x);
   TORCH_CHECK(version >= 0 && version <= 5, "version must be 0..5");
   TORCH_CHECK(split_k >= 1 && split_k <= 32, "split_k must be in [1, 32]");
@@ -234,8 +234,9 @@ void check_gate_up(const torch::Tensor& gate, const torch::Tensor& gate_scales,
 
 // h = fp16(silu(gate x) * (up x)): the fused gate/up projection of an MLP
 // decode step. No counterpart in the reference (it composes its gemv).
-torch::Tensor gate_up_silu(torch::Tensor gate, torch::Tensor gate_scales, torch::Tensor up,
-                           torch::Tensor up_scales, torch::Tensor x) {
+torch::Tensor gate_up_silu(const torch::Tensor& gate, const torch::Tensor& gate_scales,
+                           const torch::Tensor& up, const torch::Tensor& up_scales,
+                           const torch::Tensor& x) {
   check_gate_up(gate, gate_scales, up, up_scales, x);
   const int I = static_cast<int>(gate.size(0));
   const int H = static_cast<int>(gate.size(1) * kNibblesPerWord);
@@ -251,9 +252,10 @@ torch::Tensor gate_up_silu(torch::Tensor gate, torch::Tensor gate_scales, torch:
 }
 
 // y = down fp16(silu(gate x) * (up x)): one MLP decode step, two launches.
-torch::Tensor mlp_decode(torch::Tensor gate, torch::Tensor gate_scales, torch::Tensor up,
-                         torch::Tensor up_scales, torch::Tensor down, torch::Tensor down_scales,
-                         torch::Tensor x) {
+torch::Tensor mlp_decode(const torch::Tensor& gate, const torch::Tensor& gate_scales,
+                         const torch::Tensor& up, const torch::Tensor& up_scales,
+                         const torch::Tensor& down, const torch::Tensor& down_scales,
+                         const torch::Tensor& x) {
   check_gate_up(gate, gate_scales, up, up_scales, x);
   const int I = static_cast<int>(gate.size(0));
   const int H = static_cast<int>(gate.size(1) * kNibblesPerWord);
@@ -325,7 +327,8 @@ torch::Tensor unpack_paired(torch::Tensor paired) {
 }
 
 // The v5 GEMV on paired weights (stamp 25); checks as w4a16_gemv.
-torch::Tensor w4a16_gemv_paired(torch::Tensor paired, torch::Tensor scales, torch::Tensor x) {
+torch::Tensor w4a16_gemv_paired(const torch::Tensor& paired, const torch::Tensor& scales,
+                                const torch::Tensor& x) {
   check_gemv_inputs(paired, scales, x);
   const int M = static_cast<int>(paired.size(0));
   const int K = static_cast<int>(paired.size(1) * kNibblesPerWord);

@@ -18,6 +18,7 @@ from typing import Optional
 
 import torch
 
+from ._native import ext as _ext
 from .layout import gemv_paired, repack_paired, unpack_paired
 from .mlp import QuantizedMLP, gate_up_silu, mlp_decode
 from .quantize import GROUP_SIZE, dequantize, quantize_and_pack
@@ -47,17 +48,6 @@ def cuda_available() -> bool:
     except Exception:
         return False
     return True
-
-
-def _ext():
-    try:
-        from . import _cuda
-    except ImportError as exc:  # fail loudly: no fallback path exists
-        raise ImportError(
-            "decode_kernel._cuda is not built; run "
-            "`python decode-kernel_amd/build_ext.py` (hipcc, gfx950)"
-        ) from exc
-    return _cuda
 
 
 def gemv(
@@ -99,12 +89,6 @@ def w4a16_linear(
         split_k = 4 if version == 4 else 1
     if reuse_weights is None:
         reuse_weights = x.dim() == 2 and x.size(0) > 1
-    return gemv(
-        packed,
-        scales,
-        x,
-        version=version,
-        split_k=split_k,
-        reuse_weights=reuse_weights,
-        warps_per_row=1,
-    )
+    if x.dim() == 1:
+        x = x.unsqueeze(0)
+    return _ext().w4a16_gemv(packed, scales, x, int(version), int(split_k), bool(reuse_weights), 1)

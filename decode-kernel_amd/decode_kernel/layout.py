@@ -17,15 +17,11 @@ from __future__ import annotations
 
 import torch
 
+from ._native import ext as _ext
+
 __all__ = ["PAIRED_STAMP", "gemv_paired", "repack_paired", "unpack_paired"]
 
 PAIRED_STAMP = 25
-
-
-def _ext():
-    from . import _ext as ext
-
-    return ext()
 
 
 def repack_paired(packed: torch.Tensor) -> torch.Tensor:

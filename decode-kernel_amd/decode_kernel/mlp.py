@@ -16,15 +16,10 @@ from dataclasses import dataclass
 
 import torch
 
+from ._native import ext as _ext
 from .quantize import quantize_and_pack
 
 __all__ = ["QuantizedMLP", "gate_up_silu", "mlp_decode"]
-
-
-def _ext():
-    from . import _ext as ext
-
-    return ext()
 
 
 def _batch(x: torch.Tensor) -> tuple[torch.Tensor, bool]:
