@@ -31,12 +31,12 @@
 // (28672 x 8192, B = 2048: 58% of the MFMA slots, 1170 TFLOP/s at 1.77 GHz;
 // a fp16 library product of that shape 1270-1390 at 1.6 GHz).
 //
-// Measured (us; before: the tiles of gemv_reuse_pfb, and for gate/up those of
-// gate_up_silu_tiles_lds):
-//   M = 28672, K = 8192:  B = 2048 820 (1970)   B = 1000 466 (1002)  B = 128 68 (150)
-//   M = K = 4096:         B = 1000 38 (82)      B = 256 15.4 (22.0)
-//   M = 11008, K = 4096:  B = 512 60 (124)      B = 128 21.5 (39.4)  B = 24 11.1 (14.0)
-//   M = 5000, K = 4224:   B = 512 36 (110)      B = 128 14.5 (34.0)  B = 20 10.6 (12.4)
+// Measured (us, cold weights; before: the 16-row tiles of gemv_reuse_pfb or
+// gemv_reuse_lds, and for gate/up those of gate_up_silu_tiles_lds):
+//   M = 28672, K = 8192:  B = 2048 820 (1970)   B = 1000 466 (1002)  B = 128 70 (143)
+//   M = K = 4096:         B = 1000 38 (82)      B = 256 16.2 (20.5)
+//   M = 11008, K = 4096:  B = 512 60 (124)      B = 128 22.8 (37.7)  B = 32 13.5 (14.1)
+//   M = 5000, K = 4224:   B = 512 36 (110)      B = 128 16.6 (33.1)  B = 17 8.6 (11.7)
 //   gate/up, I = 11008, H = 4096: B = 512 113 (365)  B = 64 22.5 (46.8)
 //   gate/up, I = 28672, H = 8192: B = 256 240 (1012) B = 32 71 (130)
 #pragma once
