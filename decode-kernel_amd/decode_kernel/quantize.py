@@ -26,6 +26,7 @@ import torch.autograd.forward_ad as fwAD
 
 GROUP_SIZE = 128
 NIBBLES_PER_WORD = 8
+INT32_MAX = 2**31 - 1
 QMIN, QMAX = -7, 7
 SCALE_FLOOR = 1e-8
 
@@ -127,6 +128,8 @@ def _plain_gpu(packed: torch.Tensor, scales: torch.Tensor):
     if not (scales.device == packed.device and scales.dtype == torch.float16
             and scales.shape == (m, groups) and scales.is_contiguous() and m * groups > 0):
         return None
+    if m > INT32_MAX or groups > INT32_MAX // GROUP_SIZE:
+        return None  # the C ABI's M and K are int
     try:
         from . import _cuda
     except ImportError:  # as before the extension is built

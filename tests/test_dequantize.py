@@ -64,3 +64,19 @@ def test_calls_that_stay_with_torch():
         assert torch.equal(dequantize(packed, s), ref)
     param = torch.nn.Parameter(scales, requires_grad=False)
     assert _plain_gpu(packed, param) is not None and torch.equal(dequantize(packed, param), ref)
+
+
+def test_rows_past_int32():
+    """K = 2^31, one more than the C ABI's int holds: torch's formulation, as
+    before the kernel, with the bits that the kernel gives for each half."""
+    words = 2**28
+    g = torch.Generator(device="cuda").manual_seed(5)
+    packed = torch.randint(-2**31, 2**31 - 1, (1, words), device="cuda", generator=g, dtype=torch.int32)
+    scales = torch.rand(1, words // 16, device="cuda", generator=g).half()
+    assert _plain_gpu(packed, scales) is None
+    w = dequantize(packed, scales, dtype=torch.float16)
+    assert w.shape == (1, 2**31)
+    for p, s, half in zip(packed.chunk(2, 1), scales.chunk(2, 1), w.chunk(2, 1)):
+        p, s = p.contiguous(), s.contiguous()
+        assert _plain_gpu(p, s) is not None
+        assert torch.equal(dequantize(p, s, dtype=torch.float16), half)
