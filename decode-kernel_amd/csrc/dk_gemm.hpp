@@ -96,21 +96,26 @@ __device__ __forceinline__ u32x4_t gemm_rsrc(const char* base, uint32_t bytes) {
 // register. m0 holds the wave's LDS byte address; lane l's 16 bytes land at
 // 16 l past it, a zero-extended halfword at 4 l. The five wait states cover
 // an SGPR of the descriptor that a vector instruction wrote just before (the
-// compiler does not look into the block).
+// compiler does not look into the block). m0 is a clobber: without it the
+// compiler keeps an address that it has in m0 for a builtin load past the
+// block. It warns that m0 is a reserved register, one that it does not save.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 template <int kOffset>
 __device__ __forceinline__ void dma16(uint32_t lds, uint32_t voff, u32x4_t r) {
   asm volatile(
       "s_add_u32 m0, %0, %3\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds),
       "v"(voff), "s"(r), "i"(kOffset)
-      : "memory", "scc");
+      : "memory", "scc", "m0");
 }
 template <int kOffset>
 __device__ __forceinline__ void dma2(uint32_t lds, uint32_t voff, u32x4_t r) {
   asm volatile(
       "s_add_u32 m0, %0, %3\n\ts_nop 3\n\tbuffer_load_ushort %1, %2, 0 offen lds" ::"s"(lds),
       "v"(voff), "s"(r), "i"(kOffset)
-      : "memory", "scc");
+      : "memory", "scc", "m0");
 }
+#pragma clang diagnostic pop
 
 // Waits until at most N of the wave's loads are in flight and its LDS reads
 // are done, and, where waves share the staged x, for the others: every wave's

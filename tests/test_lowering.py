@@ -70,3 +70,44 @@ def test_agent_scope_atomics_bypass_the_l2(tmp_path):
                      body)
     # No L2 write-back or invalidate: the relaxed form costs nothing extra.
     assert "buffer_wbl2" not in body and "buffer_inv" not in body
+
+
+# The many-batch kernel's loads to LDS (dk_gemm.hpp: dma16, dma2) set m0 in an
+# asm block. A builtin load to LDS keeps its own address there, so it has to
+# set m0 again after such a block.
+DMA_SNIPPET = r"""
+#include "dk_gemm.hpp"
+extern "C" __global__ void builtin_around_dma(const uint4* p, uint32_t bytes, uint32_t* out) {
+  __shared__ uint4 a[64], b[128];
+  const auto r = __builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, bytes, 0x00020000);
+  const uint32_t lane = threadIdx.x;
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (dk::lds_void_ptr)a, 16, lane * 16, 0, 0, 0);
+  dk::dma16<0>(dk::lds_address(b), lane * 16, dk::gemm_rsrc((const char*)p, bytes));
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (dk::lds_void_ptr)a, 16, lane * 16, 1024, 0, 0);
+  dk::dma2<0>(dk::lds_address(b + 64), lane * 2, dk::gemm_rsrc((const char*)p, bytes));
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (dk::lds_void_ptr)a, 16, lane * 16, 2048, 0, 0);
+  __builtin_amdgcn_s_waitcnt(0);
+  out[lane] = a[lane].x + b[lane].x;
+}
+"""
+
+
+@pytest.mark.skipif(not HIPCC.exists(), reason="no hipcc")
+def test_lds_loads_in_asm_clobber_m0(tmp_path):
+    repo = Path(__file__).resolve().parents[1]
+    src = tmp_path / "dma.hip"
+    src.write_text(DMA_SNIPPET)
+    asm = tmp_path / "dma.s"
+    subprocess.run([str(HIPCC), "--offload-arch=gfx950", "-O3", "-std=c++17", "--cuda-device-only",
+                    "-S", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+                    f"-I{repo / 'include'}", f"-I{repo / 'decode-kernel_amd' / 'csrc'}",
+                    str(src), "-o", str(asm)], check=True, capture_output=True, timeout=300)
+    text = asm.read_text()
+    body = text[text.index("builtin_around_dma:"):]
+    body = body[:body.index("s_endpgm")]
+    loads = list(re.finditer(r"^\s*buffer_load_\w+ .*\blds$", body, re.M))
+    assert len(loads) == 5, body
+    start = 0
+    for n, load in enumerate(loads):  # every load's own m0, set since the load before it
+        assert re.search(r"^\s*s_\w+ m0,", body[start:load.start()], re.M), (n, load.group())
+        start = load.end()
