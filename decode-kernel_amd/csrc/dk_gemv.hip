@@ -495,6 +495,36 @@ GemmShape gemm_best(int M, int K, int B, bool gate_up) {
   return best;
 }
 
+// Without scale pairs: whether rows of up to 1408 weights are long enough for
+// gemm_w4. Its K parts have at most two groups each there (one part or none on
+// the shortest rows), so the 16-row tiles win where they fill the chip in few
+// rounds: up to 48 batch rows over 4096 rows, where a wave has two of them,
+// and up to 72 batch rows up to 6144 rows. us over cold weights, gemm_w4 first:
+//   K = 128: M = 5364, B = 41 7.0 (3.2), M = 1464, B = 455 7.6 (19.0);
+//            M = 2704, B = 81 3.8 (5.2), M = 114, B = 2012 3.9 (53.9);
+//            M = 35120, B = 127 9.0 (28.4)
+//   K = 384: M = 6899, B = 26 4.3 (3.8), M = 4553, B = 40 5.3 (4.0);
+//            M = 14749, B = 21 5.0 (6.0), M = 2584, B = 40 3.8 (3.5)
+//   K = 640: M = 4500, B = 57 5.9 (5.3), M = 17276, B = 28 8.4 (7.3)
+//   K = 896: M = 14982, B = 45 8.3 (9.8), M = 5459, B = 25 5.0 (4.8)
+//   K = 1152: M = 4861, B = 38 6.8 (5.4); K = 1920, M = 5955, B = 48 8.2 (9.7)
+// At 6878 drawn sizes that gemm_w4 took before these lines, 648 ran more than
+// 4% slower than on the 16-row tiles; now 48 do, and 60 others would gain 4% or
+// more from gemm_w4.
+bool short_rows_gain(int M, int K, int B) {
+  const long long t64 = ceil_div(M, 64) * ceil_div(B, 64);
+  if (K == DK_GROUP_SIZE) {
+    const bool one_round = ceil_div(M, 32) * ceil_div(B, 32) <= 256;
+    return (one_round && M <= (B > 48 ? 4096 : 2048)) || t64 > 352 || B > 192;
+  }
+  if (K <= 1024) {
+    if (B <= 32) return t64 > 192 && t64 <= 256;
+    if (B <= 48) return M <= 4096 || M > 12288;
+    return B > 72 || M <= 4096 || M > 6144;
+  }
+  return K > 1408 || B <= 32 || B > 48 || M <= 4096 || M > 5120;
+}
+
 // Where gemm_w4 takes the weight-reuse path's batches (`pairs`: the scales
 // load in pairs) and gate/up's: above 16 batch rows, where its tiles come near
 // to one per CU. Its 32-bit offsets take K up to 2^21. Against the 16-row
@@ -513,11 +543,13 @@ GemmShape gemm_best(int M, int K, int B, bool gate_up) {
 //           M = 28672, K = 8192, B = 17 43.1 (46.1);  M = 9216, B = 32 24.5 (23.3);
 //           M = 10240, K = 28672, B = 17 68.3 (65.5), 32 77.5 (68.1)
 //   no pairs (the 16-row tiles are slower there): over 512 tiles of 16 x 16, above 32 batch rows
-//           384 from 1025 rows on:
+//           384 at 1025 to 2048 rows:
 //           M = 5000, K = 4224, B = 17 8.6 (11.7), 64 12.0 (18.6);
 //           M = 3584, K = 10880, B = 17 16.7 (14.1); M = 4608 17.1 (21.4);
 //           M = 1536, K = 10880, B = 33 15.6 (13.6), 64 18.0 (19.4);
-//           M = 2048, K = 1152, B = 33 4.8 (5.9); M = 1024, K = 10880, B = 128 17.2 (16.8)
+//           M = 2048, K = 1152, B = 33 4.8 (5.9); M = 1024, K = 10880, B = 128 17.2 (16.8);
+//           M = 2534, K = 4992, B = 40 9.6 (7.0); M = 2409, K = 1920, B = 37 6.1 (5.1);
+//           and on short rows where short_rows_gain says so
 //   gate/up, likewise:
 //           I = 2048, H = 4096, B = 64 11.0 (10.2), 128 15.7 (17.7);
 //           I = 3584, H = 8192, B = 32 18.3 (19.9), 48 18.5 (28.1);
@@ -530,7 +562,8 @@ GemmShape gemm_shape(int M, int K, int B, bool pairs) {
   } else if (pairs) {
     take = K > 1024 && ceil_div(M, 32) * ceil_div(B, 32) > 256;
   } else {
-    take = ceil_div(M, 16) * ceil_div(B, 16) >= (B > 32 && M > 1024 ? 384 : 513);
+    take = ceil_div(M, 16) * ceil_div(B, 16) >= (B > 32 && M > 1024 && M <= 2048 ? 384 : 513) &&
+           short_rows_gain(M, K, B);
   }
   return take ? gemm_best(M, K, B, false) : GemmShape{};
 }

@@ -43,15 +43,40 @@ def lib():
     (1024, 8192, 257, "gemm_w4<1, 8, 2, 1, false>", 160),
     (28672, 8192, 2048, "gemm_w4<4, 1, 4, 2, false>", 1792),
     (4096, 1024, 1000, "gemv_reuse_pfb<", None),
-    # Odd group counts: over 512 tiles of 16 x 16, 384 from 1025 rows on above
-    # 32 batch rows.
+    # Odd group counts: over 512 tiles of 16 x 16, 384 at 1025 to 2048 rows
+    # above 32 batch rows.
     (4096, 4224, 32, "gemv_reuse_lds<", None),
     (4097, 4224, 32, "gemm_w4<1, 8, 1, 1, false>", 129),
     (2032, 4224, 33, "gemv_reuse", None),
     (2033, 4224, 33, "gemm_w4<1, 8, 1, 1, false>", 128),
+    (2048, 4224, 48, "gemm_w4<1, 8, 1, 1, false>", 128),
+    (2049, 4224, 33, "gemv_reuse", None),
+    (2736, 4224, 48, "gemm_w4<1, 8, 1, 1, false>", 172),
     (1024, 4224, 128, "gemv_reuse", None),
     (1024, 4224, 129, "gemm_w4<1, 8, 1, 1, false>", 160),
     (5000, 4224, 20, "gemm_w4<1, 8, 1, 1, false>", 157),
+    # Short rows, odd group counts: the 16-row tiles over 4096 rows up to 48
+    # batch rows and up to 6144 rows up to 72; with one group but for one round
+    # of 32 x 32 tiles, over 352 tiles of 64 x 64 or over 192 batch rows.
+    (4161, 384, 17, "gemv_reuse_lds<", None),
+    (12288, 640, 32, "gemv_reuse_lds<", None),
+    (12289, 640, 32, "gemm_w4<1, 8, 1, 2, false>", 193),
+    (16385, 640, 32, "gemv_reuse_lds<", None),
+    (4096, 896, 48, "gemm_w4<", None),
+    (4097, 896, 48, "gemv_reuse", None),
+    (4096, 640, 49, "gemm_w4<", None),
+    (4097, 640, 72, "gemv_reuse", None),
+    (4097, 640, 73, "gemm_w4<", None),
+    (6144, 640, 72, "gemv_reuse", None),
+    (6145, 640, 72, "gemm_w4<", None),
+    (4861, 1152, 38, "gemv_reuse", None),
+    (5121, 1408, 38, "gemm_w4<", None),
+    (5120, 1664, 38, "gemm_w4<", None),
+    (5364, 128, 41, "gemv_reuse_lds<", None),
+    (16392, 128, 64, "gemv_reuse", None),
+    (16392, 128, 129, "gemm_w4<4, 1, 4, 2, false>", 130),
+    (2704, 128, 81, "gemm_w4<1, 8, 1, 1, false>", 255),
+    (114, 128, 2012, "gemm_w4<1, 8, 1, 1, false>", 252),
     (256, 1024, 300, "gemv_reuse", None),
     (1024, 28672, 33, "gemv_reuse_pf<", None),
     (4096, 1 << 21, 65, "gemm_w4<", None),
@@ -112,15 +137,15 @@ def _check(y: torch.Tensor, ref: torch.Tensor, label: str):
 
 
 LINEAR = [
-    ((4161, 384, 17), "<1, 8, 1, 1,"), ((8191, 4224, 31), "<1, 8, 1, 1,"), ((513, 128, 250), "<1, 8, 1, 1,"),
+    ((4095, 384, 33), "<1, 8, 1, 1,"), ((8191, 4224, 31), "<1, 8, 1, 1,"), ((513, 128, 250), "<1, 8, 1, 1,"),
     ((5000, 4224, 24), "<1, 8, 1, 1,"), ((4095, 2176, 33), "<1, 8, 1, 1,"),
     ((2049, 640, 128), "<1, 8, 2, 1,"), ((4090, 4224, 65), "<1, 8, 2, 1,"),
-    ((8193, 1280, 17), "<1, 8, 1, 2,"), ((5000, 1152, 80), "<1, 8, 1, 2,"), ((8193, 640, 33), "<1, 8, 2, 2,"),
+    ((8193, 1280, 17), "<1, 8, 1, 2,"), ((5000, 1152, 80), "<1, 8, 1, 2,"), ((8193, 640, 49), "<1, 8, 2, 2,"),
     ((5000, 4224, 129), "<1, 8, 2, 2,"),
     ((16385, 640, 64), "<2, 4, 2, 2,"), ((4100, 4224, 300), "<2, 4, 2, 2,"),
     ((2040, 11136, 640), "<1, 8, 4, 2,"), ((11008, 4224, 129), "<2, 4, 4, 2,"),
     ((5000, 4224, 520), "<2, 4, 4, 2,"),
-    ((8321, 384, 33), "<1, 4, 4, 2,"), ((2049, 640, 1030), "<1, 4, 4, 2,"),
+    ((8321, 384, 65), "<1, 4, 4, 2,"), ((2049, 640, 1030), "<1, 4, 4, 2,"),
     ((16392, 128, 129), "<4, 1, 4, 2,"), ((2053, 128, 1000), "<4, 1, 4, 2,"),
 ]
 
