@@ -535,6 +535,13 @@ bool short_rows_gain(int M, int K, int B) {
 //           M = K = 4096, B = 64 9.2 (8.6), 96 11.6 (13.1), 256 16.2 (20.5);
 //           M = K = 8192, B = 48 21.0 (23.9), 128 28.8 (37.3), 256 44.0 (66.1);
 //           M = 5632, K = 28672, B = 33 56.8 (65.6), 64 66.7 (66.8);
+//           at 129 to 304 rows of over 1536 weights, whose few row tiles read a
+//           long x on every XCD, not from 321 tiles up to 128 of 64 x 64, where the 16-row tiles,
+//           four by four in a workgroup, are still one round: M = 227, K = 3584,
+//           B = 1432 16.9 (12.8); M = 253, K = 1792, B = 1865 11.6 (8.0);
+//           M = 284, K = 2304, B = 1642 (130 of 64 x 64) 12.5 (19.3);
+//           M = 272, K = 1536, B = 1176 6.4 (9.1);
+//           M = 117, K = 4608, B = 8781 24.2 (532);
 //           rows of up to 1024 weights stay (M = 4096, K = 1024, B = 64 5.3
 //           (4.7), 128 6.7 (6.7), 256 6.9 (8.7));
 //   pairs, 17 to 32 batch rows: over 8192 rows, B K up to 3 2^16, for each
@@ -560,7 +567,10 @@ GemmShape gemm_shape(int M, int K, int B, bool pairs) {
   if (pairs && B <= 32) {
     take = K > 1024 && M > 8192 && B * K <= 3 << 16;
   } else if (pairs) {
-    take = K > 1024 && ceil_div(M, 32) * ceil_div(B, 32) > 256;
+    const long long tiles = ceil_div(M, 32) * ceil_div(B, 32);
+    take = K > 1024 && tiles > 256 &&
+           !(K > 1536 && M > 128 && M <= 304 && tiles > 320 &&
+             ceil_div(M, 64) * ceil_div(B, 64) <= 128);
   } else {
     take = ceil_div(M, 16) * ceil_div(B, 16) >= (B > 32 && M > 1024 && M <= 2048 ? 384 : 513) &&
            short_rows_gain(M, K, B);

@@ -42,6 +42,16 @@ def lib():
     (1024, 8192, 256, "gemv_reuse", None),
     (1024, 8192, 257, "gemm_w4<1, 8, 2, 1, false>", 160),
     (28672, 8192, 2048, "gemm_w4<4, 1, 4, 2, false>", 1792),
+    # At 129 to 304 rows of over 1536 weights not from 321 tiles up to 128 of
+    # 64 x 64.
+    (256, 1536, 1409, "gemm_w4<", None),
+    (227, 3584, 1432, "gemv_reuse_pfb<", None),
+    (129, 4096, 2100, "gemv_reuse", None),
+    (128, 4096, 2700, "gemm_w4<", None),
+    (256, 4096, 1280, "gemm_w4<", None),
+    (304, 4096, 1600, "gemv_reuse", None),
+    (304, 4096, 1601, "gemm_w4<", None),
+    (305, 4096, 1500, "gemm_w4<", None),
     (4096, 1024, 1000, "gemv_reuse_pfb<", None),
     # Odd group counts: over 512 tiles of 16 x 16, 384 at 1025 to 2048 rows
     # above 32 batch rows.
