@@ -578,8 +578,33 @@ GemmShape gemm_shape(int M, int K, int B, bool pairs) {
   return take ? gemm_best(M, K, B, false) : GemmShape{};
 }
 
+// Gate/up: whether rows of up to 2048 weights are long enough for gemm_w4, as
+// short_rows_gain. At 512 to 2048 weights a batch tile of up to 32 rows loses
+// where the rows of I just exceed one round (64 in each of 256 workgroups). us
+// over cold weights, gemm_w4 first:
+//   H = 128: I = 2925, B = 45 7.4 (3.8); I = 4045, B = 96 10.1 (6.7);
+//            I = 12958, B = 61 8.5 (13.1);
+//   H = 512: I = 3187, B = 38 6.0 (4.1); I = 2430, B = 453 12.5 (16.7)
+//   H = 1024: I = 5052, B = 38 10.1 (7.5); I = 5702, B = 35 9.6 (8.6);
+//             H = 896, I = 16983, B = 20 17.8 (13.0)
+//   H = 1152: I = 895, B = 204 7.3 (6.3); H = 1920: I = 690, B = 180 8.6 (7.4)
+// At 5290 drawn sizes that gemm_w4 took before these lines, 1060 ran more than
+// 4% slower than on the 16-row tiles; now 59 do, and 74 others would gain 4% or
+// more from gemm_w4.
+bool gate_up_short_rows_gain(int I, int H, int B) {
+  if (H > 2048) return true;
+  const long long t16 = ceil_div(I, 16) * ceil_div(B, 16);
+  const long long t32 = ceil_div(I, 32) * ceil_div(B, 32);
+  if (H == DK_GROUP_SIZE) return ceil_div(I, 64) * ceil_div(B, 64) > 216 || t32 > 640;
+  if (H >= 512 && B <= 32 && I > 16384 && I <= (H <= 1024 ? 24576 : 18432)) return false;
+  if (H <= 1024) return t16 > 1536 || (t16 > 768 && t32 <= 256);
+  return t32 > (H <= 1792 ? 176 : 144);
+}
+
 GemmShape gate_up_gemm_shape(int I, int H, int B) {
-  if (B <= 16 || H > (1 << 21) || ceil_div(I, 16) * ceil_div(B, 16) <= 512) return {};
+  if (B <= 16 || H > (1 << 21) || ceil_div(I, 16) * ceil_div(B, 16) <= 512 ||
+      !gate_up_short_rows_gain(I, H, B))
+    return {};
   return gemm_best(I, H, B, true);
 }
 

@@ -107,6 +107,29 @@ def test_linear_routes(lib, m, k, b, kernel, blocks):
     (2048, 4096, 65, "gemm_w4<1, 8, 1, 2, true>"),
     (11008, 4096, 1000, "gemm_w4<4, 1, 4, 2, true>"),
     (512, 4096, 20, "gate_up_silu_"),
+    # Short rows: up to 1024 weights over 1536 tiles of 16 x 16, or over 768 in
+    # one round of 32 x 32; up to 2048 over 144 or 176 of 32 x 32; one group
+    # over 216 of 64 x 64 or 640 of 32 x 32.
+    (4100, 256, 17, "gate_up_silu_tiles_lds"),
+    (4096, 1024, 96, "gate_up_silu_tiles_lds"),
+    (4097, 1024, 96, "gemm_w4"),
+    (4096, 512, 64, "gemm_w4"),
+    (3072, 512, 64, "gate_up_silu_tiles_lds"),
+    (4128, 512, 64, "gate_up_silu_tiles_lds"),
+    (2816, 1152, 64, "gate_up_silu_tiles_lds"),
+    (2817, 1152, 64, "gemm_w4"),
+    (2304, 2048, 64, "gate_up_silu_tiles_lds"),
+    (2305, 2048, 64, "gemm_w4"),
+    (2304, 2176, 64, "gemm_w4"),
+    (16384, 512, 32, "gemm_w4"),
+    (16385, 512, 32, "gate_up_silu_tiles_lds"),
+    (24577, 512, 32, "gemm_w4"),
+    (16385, 384, 32, "gemm_w4"),
+    (18433, 2048, 32, "gemm_w4"),
+    (13824, 128, 32, "gate_up_silu_tiles_lds"),
+    (13825, 128, 32, "gemm_w4<4, 1, 4, 2, true>"),
+    (10240, 128, 64, "gate_up_silu_tiles_lds"),
+    (10241, 128, 64, "gemm_w4<4, 1, 4, 2, true>"),
 ])
 def test_gate_up_routes(lib, i, h, b, kernel):
     assert _abi.describe_gate_up(lib, i, h, b)["kernel"].startswith("void dk::" + kernel)
@@ -221,10 +244,11 @@ def test_linear_least_alignment(lib, shape):
 
 
 GATE_UP = [
-    ((4100, 256, 17), "<1, 8, 1, 2,"), ((1000, 384, 250), "<1, 8, 1, 2,"), ((4100, 640, 33), "<1, 8, 2, 2,"),
-    ((2049, 640, 128), "<1, 8, 2, 2,"), ((8193, 384, 17), "<2, 4, 2, 2,"), ((8193, 4224, 65), "<2, 4, 4, 2,"),
-    ((4100, 256, 33), "<1, 4, 4, 2,"), ((3000, 384, 250), "<1, 4, 4, 2,"), ((4100, 128, 17), "<4, 1, 4, 2,"),
-    ((1000, 128, 513), "<4, 1, 4, 2,"), ((2049, 128, 129), "<4, 1, 4, 2,"), ((5888, 13184, 70), "<1, 8, 4, 2,"),
+    ((5633, 1152, 17), "<1, 8, 1, 2,"), ((1000, 384, 250), "<1, 8, 1, 2,"), ((4100, 1152, 33), "<1, 8, 2, 2,"),
+    ((2049, 1152, 128), "<1, 8, 2, 2,"), ((8193, 1152, 17), "<2, 4, 2, 2,"), ((8193, 384, 33), "<2, 4, 2, 2,"),
+    ((8193, 4224, 65), "<2, 4, 4, 2,"), ((4100, 256, 97), "<1, 4, 4, 2,"), ((3000, 384, 250), "<1, 4, 4, 2,"),
+    ((13825, 128, 17), "<4, 1, 4, 2,"), ((1000, 128, 2100), "<4, 1, 4, 2,"), ((2049, 128, 449), "<4, 1, 4, 2,"),
+    ((5888, 13184, 70), "<1, 8, 4, 2,"),
 ]
 
 
