@@ -23,6 +23,7 @@ from __future__ import annotations
 
 import torch
 import torch.autograd.forward_ad as fwAD
+from torch.utils._device import DeviceContext
 
 GROUP_SIZE = 128
 NIBBLES_PER_WORD = 8
@@ -114,8 +115,10 @@ def _plain_gpu(packed: torch.Tensor, scales: torch.Tensor):
         return None  # other subclasses (fake tensors) keep their own dispatch
     if torch.compiler.is_compiling() or torch.jit.is_tracing():
         return None
-    if torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack():
-        return None
+    if torch._C._len_torch_dispatch_stack() or not all(
+            type(torch._C._get_function_stack_at(i)) is DeviceContext
+            for i in range(torch._C._len_torch_function_stack())):
+        return None  # a default device only tells where new tensors go
     wrapped = torch._C._functorch.is_functorch_wrapped_tensor
     if wrapped(packed) or wrapped(scales) or scales.is_neg():
         return None

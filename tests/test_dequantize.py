@@ -66,6 +66,29 @@ def test_calls_that_stay_with_torch():
     assert _plain_gpu(packed, param) is not None and torch.equal(dequantize(packed, param), ref)
 
 
+def test_under_a_default_device():
+    """torch.set_default_device leaves a function mode on the stack for the whole
+    process: it keeps the HIP pass; any other mode sees torch's operations."""
+    packed, scales = _case(16, 256, seed=2)
+    scales = torch.rand_like(scales)
+    ref = dequantize_torch(packed, scales)
+    for device in ("cuda", "cpu"):
+        with torch.device(device):
+            assert _plain_gpu(packed, scales) is not None
+            assert torch.equal(dequantize(packed, scales), ref)
+    seen = []
+
+    class Watch(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    with torch.device("cuda"), Watch():
+        assert _plain_gpu(packed, scales) is None
+        out = dequantize(packed, scales)
+    assert seen and torch.equal(out, ref)
+
+
 def test_rows_past_int32():
     """K = 2^31, one more than the C ABI's int holds: torch's formulation, as
     before the kernel, with the bits that the kernel gives for each half."""
