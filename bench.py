@@ -31,7 +31,7 @@ Also reported on the same line: the read roof (best 1 GiB STREAM read), the
 copy roof, the read floor (the fastest launch shape of a kernel that only
 reads the headline's bytes), the empty-kernel timing floors, every kernel
 variant at the headline shape, the other four configurations, a roofline
-object for the headline kernel (named by dk_gemv_describe), the fp16 GEMM
+object for the headline kernel (named by the dispatch itself), the fp16 GEMM
 ridge point, and the CPU baseline: the reference's CPU path (fp32
 dequantize + F.linear, python/decode_kernel/reference.py:17-26) in torch on
 this host's cores.
@@ -464,10 +464,10 @@ def c3_crossover(results: dict, margin: float):
 
 
 def kernel_of(m, k, b, **cfg):
-    """The kernel the C ABI dispatches for this call (dk_gemv_describe)."""
+    """The kernel that the timed extension call with these keywords launches."""
     from decode_kernel import _abi
 
-    return _abi.describe(_abi.load(), m, k, b, **{kk: int(v) for kk, v in cfg.items()})
+    return _abi.describe_extension(_abi.load(), m, k, b, **cfg)
 
 
 def profiled_traffic(kernel: str):

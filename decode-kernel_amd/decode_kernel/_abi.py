@@ -170,6 +170,14 @@ def describe_linear(lib: ctypes.CDLL, m: int, k: int, b: int) -> dict:
     return _launch(info)
 
 
+def describe_extension(lib: ctypes.CDLL, m: int, k: int, b: int, **config) -> dict:
+    """The kernel the torch extension's w4a16_gemv launches for these keywords:
+    with reuse_weights it calls dk_w4a16_linear, else dk_w4a16_gemv."""
+    if config.get("reuse_weights"):
+        return describe_linear(lib, m, k, b)
+    return describe(lib, m, k, b, **config)
+
+
 def describe_gate_up(lib: ctypes.CDLL, i: int, h: int, b: int) -> dict:
     """The kernel dk_gate_up_silu would launch."""
     info = LaunchInfo()

@@ -66,7 +66,7 @@ def main() -> None:
         xd = torch.from_numpy(x).cuda()
         n = len(pk)
         kw = dict(reuse_weights=True) if b > 1 else {}
-        kernel = _abi.describe(lib, m, k, b, **{kk: int(v) for kk, v in kw.items()})["kernel"]
+        kernel = _abi.describe_extension(lib, m, k, b, **kw)["kernel"]
         g, graph = time_graph_steps(lambda i: gemv(pk[i % n], sc[i % n], xd, **kw),
                                     steps=args.steps, preroll=flush)
         del graph

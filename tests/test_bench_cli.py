@@ -1,6 +1,7 @@
 """bench.py's command-line contract that needs no GPU: it measures one GPU
 only, so any other --gpus (or a WORLD_SIZE above 1) exits with status 2 and a
-message before touching a device."""
+message before touching a device. And the kernel that it names beside a time
+is the one that the timed call launches."""
 
 from __future__ import annotations
 
@@ -37,3 +38,15 @@ def test_help_lists_the_contract_flags():
     assert out.returncode == 0
     for flag in ("--gpus", "--steps", "--warmup"):
         assert flag in out.stdout
+
+
+def test_kernel_names_are_those_of_the_timed_calls():
+    # The extension sends reuse_weights to dk_w4a16_linear, which has the
+    # many-batch kernel; the streaming variants go to dk_w4a16_gemv.
+    import bench
+
+    for b, kernel in ((16, "gemv_reuse_pf<"), (64, "gemv_reuse"), (128, "gemm_w4<1, 8, 2, 1, false>"),
+                      (256, "gemm_w4<1, 8, 2, 2, false>")):
+        assert kernel in bench.kernel_of(4096, 4096, b, **bench.VARIANTS["reuse"])["kernel"], b
+    assert "gemv_v5_lds<" in bench.kernel_of(4096, 4096, 1, **bench.VARIANTS["v5"])["kernel"]
+    assert "gemv_v1_multiwave" in bench.kernel_of(4096, 4096, 1, **bench.VARIANTS["v1_wpr4"])["kernel"]
