@@ -243,6 +243,29 @@ def test_linear_least_alignment(lib, shape):
     _check(y.view(b, m), x.double() @ _dense(packed, scales).T, f"{m}x{k} B={b}")
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(4161, 384, 17), (5000, 4224, 24), (8200, 1280, 70),
+                                   (4096, 4096, 100)])
+def test_linear_agrees_with_gemv(lib, shape):
+    """dk_w4a16_gemv keeps the 16-row tiles: the same bits where dk_w4a16_linear
+    does too, else both within their bound (fp32 sums in another order)."""
+    m, k, b = shape
+    packed, scales = _weight(m, k, seed=m + b)
+    x = _x(b, k, seed=b)
+    cfg = _abi.default_config(lib, reuse_weights=1)
+    y = torch.empty(2, b, m, dtype=torch.float16, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    args = (packed.data_ptr(), scales.data_ptr(), x.data_ptr())
+    _abi.check(lib, lib.dk_w4a16_gemv(*args, y[0].data_ptr(), m, k, b, ctypes.byref(cfg), None, 0,
+                                      stream))
+    _abi.check(lib, lib.dk_w4a16_linear(*args, y[1].data_ptr(), m, k, b, None, 0, stream))
+    if _abi.describe_linear(lib, m, k, b) == _abi.describe(lib, m, k, b, reuse_weights=1):
+        assert torch.equal(y[0], y[1])
+    ref = x.double() @ _dense(packed, scales).T
+    for out, entry in zip(y, ("gemv", "linear")):
+        _check(out, ref, f"{entry} {m}x{k} B={b}")
+
+
 GATE_UP = [
     ((5633, 1152, 17), "<1, 8, 1, 2,"), ((1000, 384, 250), "<1, 8, 1, 2,"), ((4100, 1152, 33), "<1, 8, 2, 2,"),
     ((2049, 1152, 128), "<1, 8, 2, 2,"), ((8193, 1152, 17), "<2, 4, 2, 2,"), ((8193, 384, 33), "<2, 4, 2, 2,"),

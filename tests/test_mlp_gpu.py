@@ -122,6 +122,28 @@ def test_gate_up_every_dispatch_class(i, h):
         _check_tight(hk.float().cpu().numpy(), h_ref[:b], f"h {i}x{h} B={b}")
 
 
+@pytest.mark.parametrize("i,h,b,kernel", [
+    (1800, 6144, 33, "gate_up_silu_tiles_lds<4, true>"),
+    (1024, 4224, 40, "gate_up_silu_tiles_lds<4, false>"),
+    (2048, 4096, 64, "gate_up_silu_tiles_lds<4, true>"),
+    (4100, 256, 33, "gate_up_silu_tiles_lds<4, true>"),
+    (2925, 128, 45, "gate_up_silu_tiles_lds<4, false>"),
+    (795, 1152, 204, "gate_up_silu_tiles_lds<4, false>"),
+])
+def test_gate_up_tiles_over_16_batch_rows(i, h, b, kernel):
+    # Two to thirteen batch tiles, the last one partial, where the many-batch
+    # kernel leaves them: few tiles, and short rows.
+    from decode_kernel import _abi, gate_up_silu
+
+    assert kernel in _abi.describe_gate_up(_abi.load(), i, h, b)["kernel"]
+    (gp, gs, up, us, _, _), (ngp, ngs, nup, nus, _, _) = _weights(i, h, seed=i + h)
+    x = _x(b, h, seed=b)
+    hk = gate_up_silu(x, gp, gs, up, us)
+    _check_tight(hk.float().cpu().numpy(),
+                 oracle.gate_up_silu_f64(x.cpu().numpy(), ngp, ngs, nup, nus), f"h {i}x{h} B={b}")
+    assert torch.equal(gate_up_silu(x, gp, gs, up, us), hk)
+
+
 def test_llama70b_full_mlp_every_row():
     # Every row of h (28672) and of y (8192), against the float64 oracle in
     # blocks of rows (the unpacked weights of the whole matrix in float64

@@ -66,6 +66,25 @@ def _gemv(packed, scales, x, **kw):
     return gemv(packed, scales, x, **kw)
 
 
+def _tiles(packed, scales, x):
+    """dk_w4a16_gemv with reuse_weights, which keeps the 16-row tiles at every
+    batch (the extension's reuse_weights goes to dk_w4a16_linear), and with the
+    workspace that it can take."""
+    from decode_kernel import _abi
+
+    lib = _abi.load()
+    m, b, k = packed.shape[0], *x.shape
+    cfg = _abi.default_config(lib, reuse_weights=1)
+    need = lib.dk_gemv_workspace_bytes(m, k, b, ctypes.byref(cfg))
+    ws = torch.empty((need + 7) // 8, dtype=torch.int64, device=x.device)
+    y = torch.empty(b, m, dtype=torch.float16, device=x.device)
+    _abi.check(lib, lib.dk_w4a16_gemv(packed.data_ptr(), scales.data_ptr(), x.data_ptr(),
+                                      y.data_ptr(), m, k, b, ctypes.byref(cfg),
+                                      ws.data_ptr() if need else None, need,
+                                      torch.cuda.current_stream().cuda_stream))
+    return y
+
+
 def _upload(w: np.ndarray, x: np.ndarray):
     packed, scales = oracle.quantize_and_pack(w)
     return (packed, scales,
@@ -197,20 +216,35 @@ def test_reuse_small_batches_run_the_streaming_kernel():
         assert "gemv_reuse_lds<" in name or "gemv_reuse_pf<" in name, (m, k, b)
 
 
-@pytest.mark.parametrize("m,k,b", [(1100, 65536, 9), (4096, 4096, 8), (4096, 11008, 5),
-                                   (8192, 28672, 8), (11008, 4096, 16), (2048, 4096, 12),
-                                   (8216, 4224, 6), (4096, 4096, 16), (3072, 8192, 4),
-                                   (8192, 16384, 3), (2048, 8192, 16), (6144, 8192, 16),
-                                   (5000, 4224, 5), (5120, 5120, 3), (3000, 8320, 16),
-                                   (4500, 5248, 12), (12000, 8320, 5), (9000, 4224, 33),
-                                   (6000, 4224, 40), (3500, 6144, 33), (1000, 4096, 12),
-                                   (4096, 4096, 4), (3000, 4096, 5), (2000, 16512, 13),
-                                   (1500, 8320, 9), (4100, 8192, 12), (4096, 11008, 32),
-                                   (1000, 16384, 33), (2040, 8192, 20), (1500, 8192, 7),
-                                   (4500, 8192, 8), (9000, 8192, 7), (11008, 4096, 3),
-                                   (14336, 8192, 2), (13900, 5120, 4), (6144, 4096, 3),
-                                   (11008, 8192, 5), (16384, 4096, 8)])
-def test_reuse_tile_kernel_exact_properties(m, k, b):
+# Every shape with the kernel that dk_w4a16_gemv runs for it.
+TILE_CASES = [
+    ((1100, 65536, 9), "gemv_reuse_pf<4, 1, 8>"), ((4096, 4096, 8), "gemv_reuse_pf<6, 1, 4>"),
+    ((4096, 11008, 5), "gemv_reuse_lds<16, 1, true, 2>"), ((8192, 28672, 8), "gemv_reuse_pf<4, 2, 4>"),
+    ((11008, 4096, 16), "gemv_reuse_lds<4, 2, true, 2>"), ((2048, 4096, 12), "gemv_reuse_pf<4, 1, 8>"),
+    ((8216, 4224, 6), "gemv_reuse<8, 2, 2, false>"), ((4096, 4096, 16), "gemv_reuse_pf<4, 1, 8>"),
+    ((3072, 8192, 4), "gemv_reuse_pf<8, 1, 4>"), ((8192, 16384, 3), "gemv_reuse_pf<4, 2, 4>"),
+    ((2048, 8192, 16), "gemv_reuse_pf<4, 1, 8>"), ((6144, 8192, 16), "gemv_reuse_pf<4, 2, 8>"),
+    ((5000, 4224, 5), "gemv_reuse_lds<8, 2, false, 2>"),
+    ((5120, 5120, 3), "gemv_reuse_lds<8, 2, true, 2>"),
+    ((3000, 8320, 16), "gemv_reuse_lds<16, 1, false, 2>"),
+    ((4500, 5248, 12), "gemv_reuse_lds<8, 2, false, 2>"),
+    ((12000, 8320, 5), "gemv_reuse<8, 2, 2, false>"),
+    ((9000, 4224, 33), "gemv_reuse_lds<4, 2, false, 2>"),
+    ((6000, 4224, 40), "gemv_reuse_lds<4, 2, false, 2>"), ((3500, 6144, 33), "gemv_reuse_pfb<4, 2, 2>"),
+    ((1000, 4096, 12), "gemv_reuse_pf<4, 1, 8>"), ((4096, 4096, 4), "gemv_reuse_pf<6, 1, 2>"),
+    ((3000, 4096, 5), "gemv_reuse_pf<6, 1, 4>"), ((2000, 16512, 13), "gemv_reuse_lds<8, 1, false, 4>"),
+    ((1500, 8320, 9), "gemv_reuse_lds<8, 1, false, 4>"), ((4100, 8192, 12), "gemv_reuse_pf<4, 2, 8>"),
+    ((4096, 11008, 32), "gemv_reuse_pf<4, 2, 8>"), ((1000, 16384, 33), "gemv_reuse_pf<4, 1, 8>"),
+    ((2040, 8192, 20), "gemv_reuse_pf<4, 1, 8>"), ((1500, 8192, 7), "gemv_reuse_pf<8, 1, 4>"),
+    ((4500, 8192, 8), "gemv_reuse_pf<4, 2, 4>"), ((9000, 8192, 7), "gemv_reuse_pf<4, 1, 4>"),
+    ((11008, 4096, 3), "gemv_reuse_pf<4, 1, 2>"), ((14336, 8192, 2), "gemv_reuse_pf<4, 2, 2>"),
+    ((13900, 5120, 4), "gemv_reuse_pf<4, 2, 2>"), ((6144, 4096, 3), "gemv_reuse_lds<8, 2, true, 2>"),
+    ((11008, 8192, 5), "gemv_reuse_pf<4, 1, 4>"), ((16384, 4096, 8), "gemv_reuse_pf<4, 2, 4>"),
+]
+
+
+@pytest.mark.parametrize("shape,kernel", TILE_CASES)
+def test_reuse_tile_kernel_exact_properties(shape, kernel):
     # The single-pass MFMA tile kernels in each of their shapes (operands
     # staged in LDS: one tile per wave with 16 or 8 waves, two tiles per wave
     # with 8 or 4 waves, the second tile partly past M at M = 8216; double
@@ -233,23 +267,27 @@ def test_reuse_tile_kernel_exact_properties(m, k, b):
     # |y| grows as sqrt(K): keep it below ~16 so the fp16 output step stays
     # inside the absolute gate (at K ~ 200000 and W ~ N(0, 0.05), |y| reaches
     # 64 and one fp16 step there is 0.06).
+    from decode_kernel import _abi
+
+    m, k, b = shape
+    assert f"dk::{kernel}(" in _abi.describe(_abi.load(), m, k, b, reuse_weights=1)["kernel"]
     w_std = 0.05 if k <= 28672 else 0.005
     w, x = oracle.make_case(m, k, b, seed=7 + b, w_std=w_std)
     packed, scales, pd, sd, xd = _upload(w, x)
-    y = _gemv(pd, sd, xd, reuse_weights=True)
-    _assert_doubles(_gemv(pd, sd, xd * 2, reuse_weights=True), y, f"reuse {m}x{k} B={b}")
-    assert torch.equal(_gemv(pd, sd, -xd, reuse_weights=True), -y)
+    y = _tiles(pd, sd, xd)
+    _assert_doubles(_tiles(pd, sd, xd * 2), y, f"reuse {m}x{k} B={b}")
+    assert torch.equal(_tiles(pd, sd, -xd), -y)
     # Each batch row alone, moved to row 0 of an otherwise zero batch of the
     # same size (same tile kernel), gives the same outputs as inside the batch.
     for j in (0, b - 1):
         xs = torch.zeros(b, k, dtype=torch.float16, device="cuda")
         xs[0] = xd[j]
-        assert torch.equal(_gemv(pd, sd, xs, reuse_weights=True)[0], y[j]), j
+        assert torch.equal(_tiles(pd, sd, xs)[0], y[j]), j
     e = torch.zeros(b, k, dtype=torch.float16, device="cuda")
     cols = [(i * 37 + 5) % k for i in range(b)]
     for i, kk in enumerate(cols):
         e[i, kk] = 1.0
-    ye = _gemv(pd, sd, e, reuse_weights=True).cpu().numpy()
+    ye = _tiles(pd, sd, e).cpu().numpy()
     for i, kk in enumerate(cols):
         q = oracle.unpack_to_int(np.ascontiguousarray(packed[:, kk // 8: kk // 8 + 1]))[:, kk % 8]
         expect = (scales[:, kk // 128].astype(np.float32) * q).astype(np.float16)
@@ -292,25 +330,25 @@ def test_reuse_many_batch_tiles(shape, kernel):
     assert kernel in _abi.describe(_abi.load(), m, k, b, reuse_weights=1)["kernel"]
     w, x = oracle.make_case(m, k, b, seed=11 + b, w_std=0.05)
     packed, scales, pd, sd, xd = _upload(w, x)
-    y = _gemv(pd, sd, xd, reuse_weights=True)
+    y = _tiles(pd, sd, xd)
     _check_against_oracle(y, oracle.linear_f64(x, packed, scales), f"pfb {m}x{k} B={b}")
-    _assert_doubles(_gemv(pd, sd, xd * 2, reuse_weights=True), y, f"pfb {m}x{k} B={b}")
-    assert torch.equal(_gemv(pd, sd, -xd, reuse_weights=True), -y)
+    _assert_doubles(_tiles(pd, sd, xd * 2), y, f"pfb {m}x{k} B={b}")
+    assert torch.equal(_tiles(pd, sd, -xd), -y)
     for j in (1, b - 1):
         xs = torch.zeros(b, k, dtype=torch.float16, device="cuda")
         xs[0] = xd[j]
-        assert torch.equal(_gemv(pd, sd, xs, reuse_weights=True)[0], y[j]), j
+        assert torch.equal(_tiles(pd, sd, xs)[0], y[j]), j
     e = torch.zeros(b, k, dtype=torch.float16, device="cuda")
     cols = [(i * 37 + 5) % k for i in range(b)]
     for i, kk in enumerate(cols):
         e[i, kk] = 1.0
-    ye = _gemv(pd, sd, e, reuse_weights=True).cpu().numpy()
+    ye = _tiles(pd, sd, e).cpu().numpy()
     for i, kk in enumerate(cols):
         q = oracle.unpack_to_int(np.ascontiguousarray(packed[:, kk // 8: kk // 8 + 1]))[:, kk % 8]
         expect = (scales[:, kk // 128].astype(np.float32) * q).astype(np.float16)
         assert np.array_equal(ye[i].view(np.uint16), expect.view(np.uint16)), (i, kk)
     # Repeated launches are bit-identical.
-    assert torch.equal(_gemv(pd, sd, xd, reuse_weights=True), y)
+    assert torch.equal(_tiles(pd, sd, xd), y)
 
 
 @pytest.mark.parametrize("m,k,b", [(4096, 4096, 8), (8192, 8192, 4), (6144, 8192, 16),
@@ -617,8 +655,7 @@ def test_random_shapes_against_oracle(m, k, b):
     if b == 1:
         paths.append(("v4", dict(version=4, split_k=4)))
     for label, kw in paths:
-        kern = _abi.describe(lib, m, k, b, reuse_weights=int(kw.get("reuse_weights", False)),
-                             version=kw.get("version", 5), split_k=kw.get("split_k", 4))["kernel"]
+        kern = _abi.describe_extension(lib, m, k, b, **kw)["kernel"]
         tag = f"{label} {m}x{k} B={b} ({kern.split('(')[0]})"
         print(f"[random] {tag}", flush=True)
         y = _gemv(pd, sd, xd, **kw)
