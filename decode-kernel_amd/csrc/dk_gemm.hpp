@@ -13,7 +13,7 @@
 // 34.4 cycles per MFMA with six, 32.3 with none; for 16x16x32, 17.4 with two
 // and 26.2 with four, so the larger shape). A group of a 64 x 128 tile takes
 // 64 MFMAs, 192 instructions to decode the weights, 128 to scale the sums and
-// about 40 for LDS and loads: 5.6 per MFMA. So:
+// about 60 for LDS, loads and addresses: 6.05 per MFMA by the counters. So:
 //   * a wave decodes its weights once for up to 128 batch rows, into 64
 //     registers that serve all of them as MFMA operands, and shares x with
 //     the waves beside it through LDS; the weights go through LDS only for
@@ -27,9 +27,10 @@
 //     workgroups of four waves per CU fall out of phase by themselves (28672 x
 //     8192, B = 2048: 811 us against 870 for one workgroup of eight waves);
 //     where a workgroup has eight waves, its second four lag by half a group.
-// The whole chip draws so much power at this load that it clocks at 1.77 GHz
-// (28672 x 8192, B = 2048: 58% of the MFMA slots, 1170 TFLOP/s at 1.77 GHz;
-// a fp16 library product of that shape 1270-1390 at 1.6 GHz).
+// What is left is idle MFMA slots, not the clock: 28672 x 8192, B = 2048 takes
+// 1.57 million cycles, of which the MFMAs fill 58% (a run with counters, 956 us:
+// 1.65 GHz, 1010 TFLOP/s; without them 820-860 us, 1120-1170). A fp16 library
+// product of that shape reaches 1270-1390 at 1.6 GHz, 76-83% of the slots.
 //
 // Measured (us, cold weights; before: the 16-row tiles of gemv_reuse_pfb or
 // gemv_reuse_lds, and for gate/up those of gate_up_silu_tiles_lds):

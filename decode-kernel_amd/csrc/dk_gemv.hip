@@ -452,8 +452,9 @@ long long ceil_div(long long a, long long b) { return (a + b - 1) / b; }
 // rounds of 256; four-wave ones two to a CU when there are more than 256, a
 // pair then taking `pair` us per step. Fitted to the shapes' times over 18
 // (M, K) from 512 x 4096 to 28672 x 8192 and six of gate/up, at batches from
-// 17 to 1000: the choice is 0.2% from the best shape on average and 5% at
-// worst. What decides is the number of workgroups: few take many K parts, few
+// 17 to 1000. Checked later at 341 sizes and up to 2048 batch rows, the choice
+// is 1.1% from the fastest shape on average, over 5% at 26 of them, and 29% at
+// worst (512 x 4096, B = 2048). What decides is the number of workgroups: few take many K parts, few
 // batch rows and one row tile each, many decode each weight for 128 batch rows
 // and leave the CU to two workgroups (us, the choice first; MT = 2 but where
 // noted; 5000 x 4224, B = 17 8.6 for <1, 8, 1, MT = 1>, 11.8 for <1, 8, 1>;
@@ -536,21 +537,24 @@ bool short_rows_gain(int M, int K, int B) {
 //           M = K = 8192, B = 48 21.0 (23.9), 128 28.8 (37.3), 256 44.0 (66.1);
 //           M = 5632, K = 28672, B = 33 56.8 (65.6), 64 66.7 (66.8);
 //           at 129 to 304 rows of over 1536 weights, whose few row tiles read a
-//           long x on every XCD, not from 321 tiles up to 128 of 64 x 64, where the 16-row tiles,
-//           four by four in a workgroup, are still one round: M = 227, K = 3584,
+//           long x on every XCD, not from 321 tiles up to 128 of 64 x 64, where
+//           the 16-row tiles, four by four in a workgroup, are still one round:
+//           M = 227, K = 3584,
 //           B = 1432 16.9 (12.8); M = 253, K = 1792, B = 1865 11.6 (8.0);
 //           M = 284, K = 2304, B = 1642 (130 of 64 x 64) 12.5 (19.3);
 //           M = 272, K = 1536, B = 1176 6.4 (9.1);
 //           M = 117, K = 4608, B = 8781 24.2 (532);
-//           rows of up to 1024 weights stay (M = 4096, K = 1024, B = 64 5.3
-//           (4.7), 128 6.7 (6.7), 256 6.9 (8.7));
+//           rows of up to 1024 weights stay. That is right only for few tiles:
+//           M = 4096, K = 1024, B = 64 5.1 (4.1), 128 6.1 (5.8), 256 7.7 (7.9),
+//           but 2048 24.9 (57.4), and M = 28672, K = 1024, B = 64 10.7 (15.7),
+//           2048 133 (393); a line between them has not been drawn yet;
 //   pairs, 17 to 32 batch rows: over 8192 rows, B K up to 3 2^16, for each
 //           workgroup stages x by itself (the 16-row tiles read it through L1):
 //           M = 8448, K = 4096, B = 17 11.9 (14.8), 32 13.2 (15.4);
 //           M = 28672, K = 8192, B = 17 43.1 (46.1);  M = 9216, B = 32 24.5 (23.3);
 //           M = 10240, K = 28672, B = 17 68.3 (65.5), 32 77.5 (68.1)
-//   no pairs (the 16-row tiles are slower there): over 512 tiles of 16 x 16, above 32 batch rows
-//           384 at 1025 to 2048 rows:
+//   no pairs (the 16-row tiles are slower there): over 512 tiles of 16 x 16,
+//           above 32 batch rows 384 at 1025 to 2048 rows:
 //           M = 5000, K = 4224, B = 17 8.6 (11.7), 64 12.0 (18.6);
 //           M = 3584, K = 10880, B = 17 16.7 (14.1); M = 4608 17.1 (21.4);
 //           M = 1536, K = 10880, B = 33 15.6 (13.6), 64 18.0 (19.4);
@@ -587,7 +591,7 @@ GemmShape gemm_shape(int M, int K, int B, bool pairs) {
 //   H = 512: I = 3187, B = 38 6.0 (4.1); I = 2430, B = 453 12.5 (16.7)
 //   H = 1024: I = 5052, B = 38 10.1 (7.5); I = 5702, B = 35 9.6 (8.6);
 //             H = 896, I = 16983, B = 20 17.8 (13.0)
-//   H = 1152: I = 895, B = 204 7.3 (6.3); H = 1920: I = 690, B = 180 8.6 (7.4)
+//   H = 1280: I = 883, B = 183 7.6 (6.0); H = 1920: I = 690, B = 180 8.6 (7.4)
 // At 5290 drawn sizes that gemm_w4 took before these lines, 1060 ran more than
 // 4% slower than on the 16-row tiles; now 59 do, and 74 others would gain 4% or
 // more from gemm_w4.

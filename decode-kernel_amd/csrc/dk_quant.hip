@@ -57,8 +57,10 @@ __global__ __launch_bounds__(256) void quantize_pack_kernel(const float4* __rest
 // Store-bound: 0.516 B read and 4 (2) B written per weight. A lane writes one
 // 16-byte piece, so that a wave's store is 1 KiB in a row, and a workgroup
 // kPieces of them 4 KiB apart, all loads before the first store. 4096 x 11008
-// to fp32: 204 MB in 29.8 us, 6.8 TB/s (a large copy reaches 4.9); torch's
-// shift, mask, convert and multiply took 535 us in ten passes.
+// to fp32: 204 MB in 29.8 us, 6.8 TB/s, where the last-level cache takes up the
+// writes; 47-48 us, 4.3 TB/s, where 600 MB of dirty lines drain meanwhile (a
+// large copy reaches 4.9). torch's shift, mask, convert and multiply took 535 us
+// in ten passes.
 constexpr int kPieces = 4;
 
 template <bool kHalf>

@@ -115,7 +115,10 @@ int dk_gemv_validate(int M, int K, int B, const dk_gemv_config* cfg);
  * Differences from the reference: launch errors are returned (the reference
  * printed and continued, csrc/gemv_w4a16.cu:9-16), and split-K is one
  * launch with a deterministic reduction inside the workgroup instead of
- * memset + atomics + convert. */
+ * memset + atomics + convert. With reuse_weights it keeps the 16-row tiles
+ * at every batch, and so do dk_w4a16_gemv_noalloc and
+ * dk_w4a16_gemv_ref_workspace: batches of over 16 rows belong to
+ * dk_w4a16_linear. */
 int dk_w4a16_gemv(const uint32_t* packed, const uint16_t* scales,
                   const uint16_t* x, uint16_t* y, int M, int K, int B,
                   const dk_gemv_config* cfg, void* workspace,
@@ -123,10 +126,14 @@ int dk_w4a16_gemv(const uint32_t* packed, const uint16_t* scales,
 
 /* The quantized F.linear for any number of batch rows: what w4a16_linear
  * (python/decode_kernel/__init__.py:62-83) computes for a batch. Arguments,
- * checks, optional workspace, stamp and results as dk_w4a16_gemv with
- * reuse_weights; above 16 batch rows it also has the many-batch kernel, which
- * decodes each weight once for up to 128 batch rows, and takes it where its
- * grid fills the chip. */
+ * checks, optional workspace and stamp as dk_w4a16_gemv with reuse_weights;
+ * above 16 batch rows it also has the many-batch kernel, which decodes each
+ * weight once for up to 128 batch rows, and takes it where its grid fills the
+ * chip: up to two to three times faster above 100 batch rows. Results agree
+ * with dk_w4a16_gemv's to the order of the fp32 sums, so the last fp16 bit may
+ * differ; up to 16 batch rows, and wherever dk_linear_describe names the same
+ * kernel as dk_gemv_describe, they are the same bits. The torch extension's
+ * reuse_weights and dk_mlp_decode's down projection come here. */
 int dk_w4a16_linear(const uint32_t* packed, const uint16_t* scales, const uint16_t* x,
                     uint16_t* y, int M, int K, int B, void* workspace, size_t workspace_bytes,
                     hipStream_t stream);
@@ -248,7 +255,9 @@ int dk_empty_kernel(hipStream_t stream);
 /* Message for the last non-DK_OK status returned on the calling thread. */
 const char* dk_last_error(void);
 
-/* ABI version of this header, (major << 16) | minor. */
+/* ABI version of this header, (major << 16) | minor. It changes with what
+ * stood before; a function that was only added does not raise it, so a loader
+ * looks such a one (dk_w4a16_linear, dk_dequantize) up by its name. */
 int dk_abi_version(void);
 #define DK_ABI_VERSION ((1 << 16) | 4)
 

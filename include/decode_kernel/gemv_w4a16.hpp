@@ -42,7 +42,8 @@ enum class KernelVersion {
 struct GemvLaunchConfig {
   KernelVersion version = KernelVersion::V5;
   int split_k = 4;             // used by v4; ignored otherwise
-  bool reuse_weights = false;  // MFMA weight-reuse path for batches
+  bool reuse_weights = false;  // 16-row MFMA tiles for batches; above 16 batch
+                               // rows dk_w4a16_linear (dk_gemv.h) is faster
   int warps_per_row = 1;       // v1 only: K split across waves of one row
 };
 
