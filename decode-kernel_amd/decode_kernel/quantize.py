@@ -115,9 +115,9 @@ def _plain_gpu(packed: torch.Tensor, scales: torch.Tensor):
         return None  # other subclasses (fake tensors) keep their own dispatch
     if torch.compiler.is_compiling() or torch.jit.is_tracing():
         return None
-    if torch._C._len_torch_dispatch_stack() or not all(
-            type(torch._C._get_function_stack_at(i)) is DeviceContext
-            for i in range(torch._C._len_torch_function_stack())):
+    modes = torch._C._len_torch_function_stack()
+    if torch._C._len_torch_dispatch_stack() or modes and not all(
+            type(torch._C._get_function_stack_at(i)) is DeviceContext for i in range(modes)):
         return None  # a default device only tells where new tensors go
     wrapped = torch._C._functorch.is_functorch_wrapped_tensor
     if wrapped(packed) or wrapped(scales) or scales.is_neg():
