@@ -496,34 +496,38 @@ GemmShape gemm_best(int M, int K, int B, bool gate_up) {
   return best;
 }
 
-// Without scale pairs: whether rows of up to 1408 weights are long enough for
+// Without scale pairs: whether rows of up to 2048 weights are long enough for
 // gemm_w4. Its K parts have at most two groups each there (one part or none on
-// the shortest rows), so the 16-row tiles win where they fill the chip in few
-// rounds: up to 48 batch rows over 4096 rows, where a wave has two of them,
-// and up to 72 batch rows up to 6144 rows. us over cold weights, gemm_w4 first:
+// the shortest rows) and its time goes in steps of a round of workgroups, where
+// the 16-row tiles' grows with their number, so the tiles win where a round
+// of gemm_w4 is far from full and they fill the chip in few rounds of their own.
+// us over cold weights, gemm_w4 first:
 //   K = 128: M = 5364, B = 41 7.0 (3.2), M = 1464, B = 455 7.6 (19.0);
 //            M = 2704, B = 81 3.8 (5.2), M = 114, B = 2012 3.9 (53.9);
-//            M = 35120, B = 127 9.0 (28.4)
+//            M = 16996, B = 44 7.5 (7.5), M = 20352, B = 51 6.7 (9.9)
 //   K = 384: M = 6899, B = 26 4.3 (3.8), M = 4553, B = 40 5.3 (4.0);
 //            M = 14749, B = 21 5.0 (6.0), M = 2584, B = 40 3.8 (3.5)
-//   K = 640: M = 4500, B = 57 5.9 (5.3), M = 17276, B = 28 8.4 (7.3)
-//   K = 896: M = 14982, B = 45 8.3 (9.8), M = 5459, B = 25 5.0 (4.8)
-//   K = 1152: M = 4861, B = 38 6.8 (5.4); K = 1920, M = 5955, B = 48 8.2 (9.7)
-// At 6878 drawn sizes that gemm_w4 took before these lines, 648 ran more than
-// 4% slower than on the 16-row tiles; now 48 do, and 60 others would gain 4% or
+//   K = 640, a round of 128 x 64 tiles up to M = 32768 at B = 32:
+//            M = 20480 8.0 (8.1), 28672 8.6 (10.8), 36864 15.1 (12.7), 49152 15.5 (16.3)
+//   K = 640: M = 4500, B = 57 5.9 (5.3); M = 10496, B = 48 6.9 (6.5), 11392 7.0 (7.7);
+//            M = 4864, B = 72 5.5 (4.8), 4992 5.5 (6.0), 5376 5.5 (6.0), 5504 6.9 (6.3)
+//   K = 1664, B = 48: M = 5376 7.5 (6.3), 5632 7.5 (7.8);  K = 2176, M = 5632 8.1 (9.9)
+// Of 3000 drawn sizes that gemm_w4 took before these lines, 296 ran more than
+// 4% slower than on the 16-row tiles; now 15 do, and 20 others would gain 4% or
 // more from gemm_w4.
 bool short_rows_gain(int M, int K, int B) {
   const long long t64 = ceil_div(M, 64) * ceil_div(B, 64);
   if (K == DK_GROUP_SIZE) {
     const bool one_round = ceil_div(M, 32) * ceil_div(B, 32) <= 256;
-    return (one_round && M <= (B > 48 ? 4096 : 2048)) || t64 > 352 || B > 192;
+    return (one_round && M <= (B > 48 ? 4096 : 2048)) || t64 > (B > 32 && B <= 64 ? 296 : 352) ||
+           B > 192;
   }
   if (K <= 1024) {
-    if (B <= 32) return t64 > 192 && t64 <= 256;
-    if (B <= 48) return M <= 4096 || M > 12288;
-    return B > 72 || M <= 4096 || M > 6144;
+    if (B <= 32) return (t64 > 192 && t64 <= 256) || (t64 > 336 && t64 <= 512) || t64 > 704;
+    if (B <= 48) return M <= 4096 || M > 10880;
+    return B > 72 || M <= 4096 || M > 6144 || (B > 64 && M > 4864 && M <= 5440);
   }
-  return K > 1408 || B <= 32 || B > 48 || M <= 4096 || M > 5120;
+  return K > 2048 || B <= 32 || B > 48 || M <= 4096 || M > 5440;
 }
 
 // Where gemm_w4 takes the weight-reuse path's batches (`pairs`: the scales
@@ -592,8 +596,8 @@ GemmShape gemm_shape(int M, int K, int B, bool pairs) {
 //   H = 1024: I = 5052, B = 38 10.1 (7.5); I = 5702, B = 35 9.6 (8.6);
 //             H = 896, I = 16983, B = 20 17.8 (13.0)
 //   H = 1280: I = 883, B = 183 7.6 (6.0); H = 1920: I = 690, B = 180 8.6 (7.4)
-// At 5290 drawn sizes that gemm_w4 took before these lines, 1060 ran more than
-// 4% slower than on the 16-row tiles; now 59 do, and 74 others would gain 4% or
+// Of 2100 drawn sizes that gemm_w4 took before these lines, 297 ran more than
+// 4% slower than on the 16-row tiles; now 21 do, and 30 others would gain 4% or
 // more from gemm_w4.
 bool gate_up_short_rows_gain(int I, int H, int B) {
   if (H > 2048) return true;

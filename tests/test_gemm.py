@@ -65,25 +65,46 @@ def lib():
     (1024, 4224, 128, "gemv_reuse", None),
     (1024, 4224, 129, "gemm_w4<1, 8, 1, 1, false>", 160),
     (5000, 4224, 20, "gemm_w4<1, 8, 1, 1, false>", 157),
-    # Short rows, odd group counts: the 16-row tiles over 4096 rows up to 48
-    # batch rows and up to 6144 rows up to 72; with one group but for one round
-    # of 32 x 32 tiles, over 352 tiles of 64 x 64 or over 192 batch rows.
+    # Short rows, odd group counts: up to 32 batch rows gemm_w4 from two thirds
+    # of a round of its launch shape on; from 33 to 48 the 16-row tiles over
+    # 4096 rows up to 10880 (5440 on rows of over 1024 weights), to 72 up to
+    # 6144; with one group but for one round of 32 x 32 tiles, over 352 tiles of
+    # 64 x 64 (296 from 33 to 64 batch rows) or over 192 batch rows.
     (4161, 384, 17, "gemv_reuse_lds<", None),
     (12288, 640, 32, "gemv_reuse_lds<", None),
     (12289, 640, 32, "gemm_w4<1, 8, 1, 2, false>", 193),
     (16385, 640, 32, "gemv_reuse_lds<", None),
+    (21504, 640, 32, "gemv_reuse_lds<", None),
+    (21505, 640, 32, "gemm_w4<2, 4, 2, 2, false>", 169),
+    (32768, 640, 17, "gemm_w4<2, 4, 2, 2, false>", 256),
+    (32769, 640, 17, "gemv_reuse_lds<", None),
+    (45056, 384, 24, "gemv_reuse_lds<", None),
+    (45057, 384, 24, "gemm_w4<", None),
     (4096, 896, 48, "gemm_w4<", None),
     (4097, 896, 48, "gemv_reuse", None),
+    (10880, 896, 48, "gemv_reuse_lds<", None),
+    (10881, 896, 48, "gemm_w4<", None),
     (4096, 640, 49, "gemm_w4<", None),
     (4097, 640, 72, "gemv_reuse", None),
     (4097, 640, 73, "gemm_w4<", None),
+    (4864, 640, 72, "gemv_reuse", None),
+    (4865, 640, 65, "gemm_w4<1, 8, 1, 2, false>", 231),
+    (5440, 640, 72, "gemm_w4<1, 8, 1, 2, false>", 255),
+    (5441, 640, 65, "gemv_reuse", None),
+    (5000, 640, 64, "gemv_reuse", None),
     (6144, 640, 72, "gemv_reuse", None),
     (6145, 640, 72, "gemm_w4<", None),
     (4861, 1152, 38, "gemv_reuse", None),
-    (5121, 1408, 38, "gemm_w4<", None),
-    (5120, 1664, 38, "gemm_w4<", None),
+    (5440, 1408, 38, "gemv_reuse_lds<", None),
+    (5441, 1408, 38, "gemm_w4<", None),
+    (5376, 1920, 48, "gemv_reuse_lds<", None),
+    (5376, 2176, 48, "gemm_w4<", None),
     (5364, 128, 41, "gemv_reuse_lds<", None),
     (16392, 128, 64, "gemv_reuse", None),
+    (18944, 128, 64, "gemv_reuse", None),
+    (18945, 128, 64, "gemm_w4<", None),
+    (22528, 128, 32, "gemv_reuse", None),
+    (22529, 128, 32, "gemm_w4<", None),
     (16392, 128, 129, "gemm_w4<4, 1, 4, 2, false>", 130),
     (2704, 128, 81, "gemm_w4<1, 8, 1, 1, false>", 255),
     (114, 128, 2012, "gemm_w4<1, 8, 1, 1, false>", 252),
@@ -175,7 +196,8 @@ LINEAR = [
     ((2049, 640, 128), "<1, 8, 2, 1,"), ((4090, 4224, 65), "<1, 8, 2, 1,"),
     ((8193, 1280, 17), "<1, 8, 1, 2,"), ((5000, 1152, 80), "<1, 8, 1, 2,"), ((8193, 640, 49), "<1, 8, 2, 2,"),
     ((5000, 4224, 129), "<1, 8, 2, 2,"),
-    ((16385, 640, 64), "<2, 4, 2, 2,"), ((4100, 4224, 300), "<2, 4, 2, 2,"),
+    ((16385, 640, 64), "<2, 4, 2, 2,"), ((21505, 640, 17), "<2, 4, 2, 2,"),
+    ((4100, 4224, 300), "<2, 4, 2, 2,"),
     ((2040, 11136, 640), "<1, 8, 4, 2,"), ((11008, 4224, 129), "<2, 4, 4, 2,"),
     ((5000, 4224, 520), "<2, 4, 4, 2,"),
     ((8321, 384, 65), "<1, 4, 4, 2,"), ((2049, 640, 1030), "<1, 4, 4, 2,"),
